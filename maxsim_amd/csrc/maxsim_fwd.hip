@@ -24,7 +24,7 @@
 //    (reference K1/K2/K3/K5/K9, maxsim.cu:70-322, 647-698, 1933-2010).  Used
 //    for padded rerank and packed pairs, whose document tiles are each used
 //    by a single query (HBM-bound), and for contrastive shapes the tiled
-//    kernel does not cover (Lq > 64).  pair_ring_kernel is its variant for
+//    kernel does not cover.  pair_ring_kernel is its variant for
 //    16-bit rows of at most 128 elements and queries of at most 64 tokens:
 //    tiles come in through two wave-private LDS slots, two tiles ahead.
 //
@@ -432,9 +432,15 @@ __global__ __launch_bounds__(256) void wide_pair_kernel(FwdArgs a) {
 // ---------------------------------------------------------------------------
 // contrastive_tiled_kernel
 // ---------------------------------------------------------------------------
-// Workgroup = 8 waves.  Wave w holds NBW query blocks: queries
-// [q0 + w*qpw, q0 + (w+1)*qpw), each of nblk = ceil(Lq/32) blocks, with
-// qpw * nblk <= NBW.  The workgroup walks the 32-row tiles of its chunk of
+// Workgroup = 8 waves, NBW query blocks each: the blocks of qpg queries of
+// nblk = ceil(Lq/32) blocks, in order (qpg * nblk <= 8 * NBW).  Where a query's
+// blocks can lie in several waves (PARTS: three blocks or more at NBW = 2), a
+// document's block sums meet in LDS.  Against pair_kernel, which streamed
+// every document from L2 once per query: 150 queries of 96 tokens x 501
+// documents of 40-512 rows, fp16, 1479 -> 510 us (339 -> 1008 TFLOP/s), the
+// same bits; what is left is the MFMA pipe, as for short queries, 15 of 16
+// blocks used and the last partial tile of every document.
+// The workgroup walks the 32-row tiles of its chunk of
 // documents in order through a ring of four LDS buffers: tile k+4 is loaded
 // straight from global memory into LDS while tile k+2's operand fragments are
 // read into registers and tile k+1's MFMAs run, so the max/argmax epilogue of
@@ -466,7 +472,7 @@ struct TiledArgs {
   int lq;
   int dim;
   int nblk;   // blocks per query
-  int qpw;    // queries per wave
+  int qpg;    // queries per workgroup (query group)
   int n_qg;   // query groups
   int n_dc;   // document chunks
   float* scores;
@@ -510,7 +516,7 @@ struct TileCursor {
   int id;         // its document index
 };
 
-template <typename T, int KS, int NBW, bool ARGMAX>
+template <typename T, int KS, int NBW, bool ARGMAX, bool PARTS>
 __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledArgs a) {
   using S = typename T::storage;
   using G = TileGeom<T, KS>;
@@ -538,13 +544,20 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
   const int dim = a.dim;
 
   // ---- query blocks of this wave -> registers
-  const int64_t q_first = ((int64_t)qg * kTiledWaves + wave) * a.qpw;
+  // block j of this wave: part blk_part[j] of query blk_q[j]; off when the
+  // group holds fewer blocks or the query does not exist
+  int64_t blk_q[NBW];
+  int blk_part[NBW];
+  bool blk_on[NBW];
   Frag<T> qf[NBW][KS];
 #pragma unroll
   for (int j = 0; j < NBW; ++j) {
-    const int64_t q = min(q_first + j / a.nblk, a.nq - 1);
-    const int part = j % a.nblk;
-    const int tok = min(part * kTileCols + c, a.lq - 1);
+    const int g = wave * NBW + j;
+    blk_q[j] = (int64_t)qg * a.qpg + g / a.nblk;
+    blk_part[j] = g % a.nblk;
+    blk_on[j] = g < a.qpg * a.nblk && blk_q[j] < a.nq;
+    const int64_t q = min(blk_q[j], a.nq - 1);
+    const int tok = min(blk_part[j] * kTileCols + c, a.lq - 1);
     const S* row = Q + (q * a.lq + tok) * (int64_t)dim;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -641,11 +654,11 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
       for (int64_t b = b_begin; b < b_end; ++b) {
 #pragma unroll
         for (int j = 0; j < NBW; ++j) {
-          const int64_t q = q_first + j / a.nblk;
-          if (j >= a.qpw * a.nblk || q >= a.nq) continue;
-          const int tok = (j % a.nblk) * kTileCols + c;
+          if (!blk_on[j]) continue;
+          const int64_t q = blk_q[j];
+          const int tok = blk_part[j] * kTileCols + c;
           if (ARGMAX && argmax_out && h == 0 && tok < a.lq) argmax_out[(q * a.nb + b) * a.lq + tok] = 0;
-          if (j % a.nblk == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
+          if (blk_part[j] == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
         }
       }
       return;
@@ -686,11 +699,11 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
       const int64_t b = __builtin_amdgcn_readfirstlane(tab_id[bl0 + __ffsll((unsigned long long)mb) - 1]);
 #pragma unroll
       for (int j = 0; j < NBW; ++j) {
-        const int64_t q = q_first + j / a.nblk;
-        if (j >= a.qpw * a.nblk || q >= a.nq) continue;
-        const int tok = (j % a.nblk) * kTileCols + c;
+        if (!blk_on[j]) continue;
+        const int64_t q = blk_q[j];
+        const int tok = blk_part[j] * kTileCols + c;
         if (ARGMAX && argmax_out && h == 0 && tok < a.lq) argmax_out[(q * a.nb + b) * a.lq + tok] = 0;
-        if (j % a.nblk == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
+        if (blk_part[j] == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
       }
     }
   }
@@ -862,7 +875,30 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
     bt[j] = -1;
     best[j] = f32x16{};
   }
-  auto epilogue = [&](f32x16 (&acc)[NBW], const TileCursor& cur) __attribute__((always_inline)) {
+  // PARTS: the part sums of the documents that ended at an even tile and
+  // the one after it, in LDS by (tile mod 4, block); done_id holds those
+  // documents (-1: none).  flush_scores(even tile) runs after the barrier that follows both tiles'
+  // epilogues in every wave, and before the next one, after which their
+  // slots are written again.  Parts are added in order, as pair_kernel does.
+  constexpr int kBlocks = kTiledWaves * NBW;
+  __shared__ float part_sums[PARTS ? 4 * kBlocks : 1];
+  int done_id[2] = {-1, -1};
+  auto flush_scores = [&](int tile) __attribute__((always_inline)) {  // tile: even
+    if (wave != ((tile >> 1) & (kTiledWaves - 1))) return;  // the waves in turn
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (done_id[i] < 0) continue;
+      const int64_t q = (int64_t)qg * a.qpg + lane;
+      if (lane < a.qpg && q < a.nq) {
+        const float* ps = part_sums + ((tile + i) & 3) * kBlocks + lane * a.nblk;
+        float sum = 0.0f;
+        for (int part = 0; part < a.nblk; ++part) sum += ps[part];
+        scores[q * a.nb + done_id[i]] = sum;
+      }
+    }
+  };
+  auto epilogue = [&](f32x16 (&acc)[NBW], const TileCursor& cur,
+                      int k_now) __attribute__((always_inline)) {
     const int valid = cur.ld - cur.t * kTileRows;
     const int row_base = cur.t * kTileRows + 4 * h;
 #pragma unroll
@@ -881,21 +917,27 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
       if (i < KS * (T::bytes == 2 ? 1 : 2)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, ARGMAX ? 5 : 2, 0);
     }
+    if (PARTS) done_id[k_now & 1] = valid <= kTileRows ? cur.id : -1;
     if (valid <= kTileRows) {  // last tile of the document
       float part_sum = 0.0f;
 #pragma unroll
       for (int j = 0; j < NBW; ++j) {
-        const int part = j % a.nblk;
-        const int64_t q = q_first + j / a.nblk;
+        const int part = blk_part[j];
+        const int64_t q = blk_q[j];
         if constexpr (ARGMAX) am[j] = best_row(best[j], m[j], bt[j]);
         merge_halves(m[j], am[j]);
         const int tok = part * kTileCols + opaque(c);
         const bool vtok = tok < a.lq;
         const float sm = half_sum(vtok ? m[j] : 0.0f);
-        part_sum = (part == 0) ? sm : part_sum + sm;
-        if ((j < a.qpw * a.nblk) && (q < a.nq)) {
+        if constexpr (PARTS) {
+          if (lane == kHalfSumLane) part_sums[(k_now & 3) * kBlocks + wave * NBW + j] = sm;
+        } else {
+          part_sum = (part == 0) ? sm : part_sum + sm;
+        }
+        if (blk_on[j]) {
           if (ARGMAX && argmax_out && h == 0 && vtok) argmax_out[(q * a.nb + cur.id) * a.lq + tok] = am[j];
-          if (part == a.nblk - 1 && lane == kHalfSumLane) scores[q * a.nb + cur.id] = part_sum;
+          if (!PARTS && part == a.nblk - 1 && lane == kHalfSumLane)
+            scores[q * a.nb + cur.id] = part_sum;
         }
         m[j] = -__builtin_inff();
         am[j] = 0;
@@ -940,15 +982,17 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
       // tiles k+2 and k+3 resident (every load of this wave landed), then
       // tiles k+4 and k+5 -> the buffers of tiles k and k+1
       wait_vm(0);
+      if constexpr (PARTS) __builtin_amdgcn_s_waitcnt(0xC07F);  // part sums written and read
       barrier();
       dma_tile(u_const, fc);
       dma_tile(std::integral_constant<int, U + 1>{}, advance(fc));
+      if constexpr (PARTS) flush_scores(k - 2);
     }
     // Past the last tile these reads and MFMAs see stale buffers; their
     // results are never used, and every wave keeps the same barrier count.
     read_frags(std::integral_constant<int, (U + 2) % kNB>{}, fr_new);
     mfma_rest(fr_nxt, acc_nxt);
-    epilogue(acc_cur, cc);
+    epilogue(acc_cur, cc, U);
     if (k + 1 >= ntiles) return true;
     // The cursor walks (scalar code with branches, document offsets read
     // from LDS) come after the MFMAs and the epilogue, off the path from
@@ -963,6 +1007,14 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
     if (step(std::integral_constant<int, 1>{})) break;
     if (step(std::integral_constant<int, 2>{})) break;
     if (step(std::integral_constant<int, 3>{})) break;
+  }
+  if constexpr (PARTS) {
+    // the documents that ended since the last barrier: the last tile's and,
+    // when it is an odd one, its predecessor's
+    if ((k & 1) == 0) done_id[1] = -1;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    barrier();
+    flush_scores(k & ~1);
   }
   // drain: no load may still be writing LDS when the workgroup exits
   __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -2135,6 +2187,30 @@ constexpr int tiled_nbw() {
   return (KS * (T::bytes == 2 ? 4 : 8) * 2 <= 64) ? 2 : 1;
 }
 
+// Document chunks for n_qg query groups, one workgroup per (group, chunk) and
+// one workgroup per CU at a time: the launch takes rounds of CUs, each as long
+// as a chunk, and every round costs a pipeline fill of kRoundTiles tiles more.
+// One round where the groups divide the CUs (C5: 32 groups, 8 chunks); with 3
+// groups, 86 chunks are 258 workgroups, a second round for two of them, where
+// 85 are one (21 queries of 64 tokens x 700 documents, bf16: 82.9 against
+// 51.5 us).
+constexpr int64_t kRoundTiles = 8;
+static int64_t chunks_for_rounds(int64_t n_qg, int64_t tiles) {
+  const int64_t cus = device_cus();
+  int64_t best = 0;
+  double best_cost = 0.0;
+  const int64_t r0 = (n_qg + cus - 1) / cus;
+  for (int64_t r = r0; r < r0 + 4; ++r) {
+    const int64_t n = r * cus / n_qg;
+    const double cost = (double)r * ((double)tiles / (double)n + (double)kRoundTiles);
+    if (best == 0 || cost < best_cost) {
+      best = n;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <typename T, int KS>
 static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   if constexpr (4 * 32 * KS * 16 * T::bytes + kDocTableBytes > 64 * 1024) {
@@ -2142,9 +2218,8 @@ static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   } else {
   constexpr int NBW = tiled_nbw<T, KS>();
   using G = TileGeom<T, KS>;
-  a.qpw = NBW / a.nblk;
-  const int64_t q_per_wg = (int64_t)a.qpw * kTiledWaves;
-  a.n_qg = (int)((a.nq + q_per_wg - 1) / q_per_wg);
+  a.qpg = kTiledWaves * NBW / a.nblk;
+  a.n_qg = (int)((a.nq + a.qpg - 1) / a.qpg);
   // About one workgroup per CU, each streaming one long tile sequence: its
   // query group against a chunk of documents holding an equal share of the
   // work (the chunks are found on the device), so every CU finishes at the
@@ -2153,7 +2228,7 @@ static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   // in the work measure).
   const int64_t w_all = a.total_d + (int64_t)kDocWork * a.nb;
   const int64_t per_table = (int64_t)kDocWork * (kMaxDocsPerGroup - 1);
-  int64_t n_dc = (device_cus() + a.n_qg - 1) / a.n_qg;
+  int64_t n_dc = chunks_for_rounds(a.n_qg, w_all / kTileRows);
   n_dc = std::max<int64_t>(n_dc, (w_all + per_table - 1) / per_table);
   n_dc = std::max<int64_t>(1, std::min<int64_t>(n_dc, a.nb));
   a.n_dc = (int)n_dc;
@@ -2164,8 +2239,10 @@ static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   // Score-only calls use the same kernel with argmax == nullptr: a variant
   // without the index search needs more registers under this schedule and
   // spills, which costs far more than the search.
-  hipLaunchKernelGGL((contrastive_tiled_kernel<T, KS, NBW, true>), grid,
-                     dim3(kTiledThreads), lds, st, a);
+  const bool in_wave = a.nblk <= NBW && NBW % a.nblk == 0;
+  hipLaunchKernelGGL((in_wave ? contrastive_tiled_kernel<T, KS, NBW, true, false>
+                              : contrastive_tiled_kernel<T, KS, NBW, true, true>),
+                     grid, dim3(kTiledThreads), lds, st, a);
   }
 }
 
@@ -2182,8 +2259,9 @@ static bool tiled_supported(int dim, int lq) {
     case 8: nbw = tiled_nbw<T, 8>(); break;
     default: nbw = tiled_nbw<T, 16>(); break;
   }
+  // a query's blocks fit one workgroup
   const int nblk = (lq + kTileCols - 1) / kTileCols;
-  return nblk <= nbw;
+  return nblk <= kTiledWaves * nbw;
 }
 
 template <typename T>
