@@ -23,8 +23,8 @@
 //    rows loaded straight from global memory into MFMA operand registers
 //    (reference K1/K2/K3/K5/K9, maxsim.cu:70-322, 647-698, 1933-2010).  Used
 //    for padded rerank and packed pairs, whose document tiles are each used
-//    by a single query (HBM-bound), and for contrastive shapes the tiled
-//    kernel does not cover.  pair_ring_kernel is its variant for
+//    by a single query (HBM-bound), and for contrastive shapes that neither
+//    the tiled kernel nor contrastive_kloop_kernel (maxsim_kloop.hip) covers.  pair_ring_kernel is its variant for
 //    16-bit rows of at most 128 elements and queries of at most 64 tokens:
 //    tiles come in through two wave-private LDS slots, two tiles ahead.
 //
@@ -37,6 +37,8 @@
 
 #include "maxsim_common.h"
 #include "maxsim_host.h"
+#include "maxsim_internal.h"
+#include "maxsim_tiled.h"
 
 namespace maxsim {
 
@@ -453,31 +455,6 @@ constexpr int kTiledThreads = kTiledWaves * 64;
 constexpr int kTileBuffers = 4;        // LDS tile ring
 constexpr int kMaxDocsPerGroup = 2048;  // LDS document list per workgroup
 constexpr int kDocTableBytes = 3 * (int)sizeof(int) * kMaxDocsPerGroup;  // rows, end, id
-constexpr int kDocWork = 32;            // work of a document beyond its rows, in rows
-constexpr int kLptKeys = 128;           // sort keys of the dealt lists: tile counts, clamped
-// Dealt lists when chunks average fewer documents than this: with 8 per
-// chunk (64 queries x 512 C5 documents) contiguous chunks of whole documents
-// hold up to 17 % more tiles than the mean (forward 139.6 -> 128.4 us
-// dealt); with 64 (C5) within 2 %, and the ranking costs more (952.7 against
-// 955 us)
-constexpr int kDealtBelowDocsPerChunk = 32;
-
-struct TiledArgs {
-  const void* q;
-  const void* d;
-  const int32_t* doff;
-  int64_t nq;
-  int64_t nb;
-  int64_t total_d;
-  int lq;
-  int dim;
-  int nblk;   // blocks per query
-  int qpg;    // queries per workgroup (query group)
-  int n_qg;   // query groups
-  int n_dc;   // document chunks
-  float* scores;
-  int32_t* argmax;
-};
 
 // One 16-byte piece per lane from global memory straight into LDS
 // (global_load_lds_dwordx4): lane i of the wave writes bytes
@@ -503,17 +480,6 @@ struct TileGeom {
   static constexpr int kPieces = kTileRows * P;             // per tile
   static constexpr int NP = (kPieces + kTiledThreads - 1) / kTiledThreads;
   static constexpr int kBufPieces = kPieces;                // uint4 per buffer
-};
-
-// Position in the (document, tile) walk of a workgroup.  All fields are
-// wave-uniform 32-bit values (document offsets are int32), so the walk stays
-// in scalar registers.
-struct TileCursor {
-  int b;          // entry of the workgroup's document list
-  int row0;       // its first row
-  int ld;         // its length (0 when past the end)
-  int t;          // tile within the document
-  int id;         // its document index
 };
 
 template <typename T, int KS, int NBW, bool ARGMAX, bool PARTS>
@@ -565,110 +531,29 @@ __global__ __launch_bounds__(kTiledThreads) void contrastive_tiled_kernel(TiledA
   }
 
   // The documents of chunk dc, as a list in LDS (rows [s, e) and index of
-  // entry bl).  Two ways to form the chunks:
-  //  * dealt (more than one chunk, fewer than kDealtBelowDocsPerChunk
-  //    documents per chunk on average, at most one document per thread):
-  //    the documents sorted by tile count, longest
-  //    first (ties by index), and dealt in snake order, place p of round r
-  //    to chunk p (r even) or n_dc - 1 - p (r odd), so every chunk gets a
-  //    near-equal share of the tiles whatever the lengths.  Every workgroup
-  //    ranks all documents itself (the same ranks everywhere): one thread
-  //    per document, RankScratch (a mask per wave and key set by LDS atomic
-  //    ORs, then a scan over the keys);
-  //  * contiguous: the documents whose work prefix W(b) = off[b] + kDocWork
-  //    * b falls in [dc, dc + 1) * W / n_dc, W = total_d + kDocWork * nb
-  //    (rows, plus one tile's worth per document for its last partial tile
-  //    and its document-end work), so chunks hold equal work, not equal
-  //    counts.  The bounds are counts of documents below each threshold, one
-  //    parallel pass over the offsets; counts partition [0, nb) for any
-  //    offsets.
+  // entry bl; see chunk_documents).
   float* __restrict__ scores = a.scores;
   int32_t* __restrict__ argmax_out = a.argmax;
   int* tab_s = reinterpret_cast<int*>(lds + kTileBuffers * G::kBufPieces);
   int* tab_e = tab_s + kMaxDocsPerGroup;
   int* tab_id = tab_e + kMaxDocsPerGroup;
-  int n_docs = 0;
-  if (a.n_dc > 1 && a.n_dc < a.nb && a.nb <= kTiledThreads &&
-      a.nb < (int64_t)kDealtBelowDocsPerChunk * a.n_dc) {
-    // scratch in the tile ring, which no load has touched yet (half the
-    // keys where the ring is small: 32-element rows)
-    constexpr int kRing = kTileBuffers * G::kBufPieces * (int)sizeof(uint4);
-    constexpr int kKeys =
-        RankScratch<kTiledWaves, kLptKeys>::kBytes <= kRing ? kLptKeys : kLptKeys / 2;
-    using Rank = RankScratch<kTiledWaves, kKeys>;
-    static_assert(Rank::kBytes <= kRing, "ranking scratch fits the tile ring");
-    const Rank rs(lds);
-    rs.clear();
-    const bool own = tid < a.nb;
-    int s0 = 0, e0 = 0, key = 0;
-    if (own) {
-      s0 = a.doff[tid];
-      e0 = a.doff[tid + 1];
-      const bool ok = (s0 >= 0) && (e0 > s0) && ((int64_t)e0 <= a.total_d);
-      const int t = ok ? (e0 - s0 + kTileRows - 1) / kTileRows : 0;
-      key = t < kKeys - 1 ? t : kKeys - 1;
-    }
-    const int r = rs.rank(own, key);
-    const int nc = a.n_dc, nbd = (int)a.nb;
-    if (own) {
-      const int rd = r / nc, p = r - rd * nc;
-      if (((rd & 1) ? nc - 1 - p : p) == dc) {
-        tab_s[rd] = s0;
-        tab_e[rd] = e0;
-        tab_id[rd] = tid;
-      }
-    }
-    const int full = nbd / nc, tail = nbd - full * nc;
-    n_docs = full + (tail > 0 && ((full & 1) ? nc - 1 - dc : dc) < tail ? 1 : 0);
-  } else {
-    __shared__ int chunk_cnt[2];
-    if (threadIdx.x < 2) chunk_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    if (a.n_dc >= a.nb) {
-      // one document per chunk: nothing to balance
-      if (threadIdx.x == 0) {
-        chunk_cnt[0] = dc;
-        chunk_cnt[1] = (int)min((int64_t)dc + 1, a.nb);
-      }
-    } else {
-      const int64_t w_all = a.total_d + (int64_t)kDocWork * a.nb;
-      const int64_t w_lo = w_all * dc / a.n_dc;
-      const int64_t w_hi = w_all * (dc + 1) / a.n_dc;
-      int c_lo = 0, c_hi = 0;
-      for (int64_t bb = threadIdx.x; bb < a.nb; bb += kTiledThreads) {
-        const int64_t w = (int64_t)a.doff[bb] + (int64_t)kDocWork * bb;
-        c_lo += w < w_lo ? 1 : 0;
-        c_hi += w < w_hi ? 1 : 0;
-      }
-      if (c_lo) atomicAdd(&chunk_cnt[0], c_lo);
-      if (c_hi) atomicAdd(&chunk_cnt[1], c_hi);
-    }
-    __syncthreads();
-    const int64_t b_begin = dc == 0 ? 0 : chunk_cnt[0];
-    const int64_t b_end = dc == a.n_dc - 1 ? a.nb : chunk_cnt[1];
-    // With non-decreasing offsets consecutive documents are kDocWork apart
-    // in W, so the host's chunk count keeps every chunk within the list.
-    // Only offsets that decrease or overrun total_d can break that; such a
-    // chunk is reported like documents with invalid offsets.
-    if (b_end - b_begin > kMaxDocsPerGroup) {
-      for (int64_t b = b_begin; b < b_end; ++b) {
+  int64_t b_begin = 0, b_end = 0;
+  const int n_docs = chunk_documents<kTiledWaves, kMaxDocsPerGroup,
+                                     kTileBuffers * G::kBufPieces * (int)sizeof(uint4)>(
+      a, dc, lds, tab_s, tab_e, tab_id, b_begin, b_end);
+  if (n_docs < 0) {
+    // a run too long for the list (broken offsets): like invalid documents
+    for (int64_t b = b_begin; b < b_end; ++b) {
 #pragma unroll
-        for (int j = 0; j < NBW; ++j) {
-          if (!blk_on[j]) continue;
-          const int64_t q = blk_q[j];
-          const int tok = blk_part[j] * kTileCols + c;
-          if (ARGMAX && argmax_out && h == 0 && tok < a.lq) argmax_out[(q * a.nb + b) * a.lq + tok] = 0;
-          if (blk_part[j] == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
-        }
+      for (int j = 0; j < NBW; ++j) {
+        if (!blk_on[j]) continue;
+        const int64_t q = blk_q[j];
+        const int tok = blk_part[j] * kTileCols + c;
+        if (ARGMAX && argmax_out && h == 0 && tok < a.lq) argmax_out[(q * a.nb + b) * a.lq + tok] = 0;
+        if (blk_part[j] == 0 && lane == 0) scores[q * a.nb + b] = __builtin_nanf("");
       }
-      return;
     }
-    n_docs = (int)(b_end - b_begin);
-    for (int i = tid; i < n_docs; i += kTiledThreads) {
-      tab_s[i] = a.doff[b_begin + i];
-      tab_e[i] = a.doff[b_begin + i + 1];
-      tab_id[i] = (int)(b_begin + i);
-    }
+    return;
   }
   // The list is in LDS once, so the tile walk never issues global loads of
   // its own: the only vector-memory loads in flight are the tile loads,
@@ -2187,30 +2072,6 @@ constexpr int tiled_nbw() {
   return (KS * (T::bytes == 2 ? 4 : 8) * 2 <= 64) ? 2 : 1;
 }
 
-// Document chunks for n_qg query groups, one workgroup per (group, chunk) and
-// one workgroup per CU at a time: the launch takes rounds of CUs, each as long
-// as a chunk, and every round costs a pipeline fill of kRoundTiles tiles more.
-// One round where the groups divide the CUs (C5: 32 groups, 8 chunks); with 3
-// groups, 86 chunks are 258 workgroups, a second round for two of them, where
-// 85 are one (21 queries of 64 tokens x 700 documents, bf16: 82.9 against
-// 51.5 us).
-constexpr int64_t kRoundTiles = 8;
-static int64_t chunks_for_rounds(int64_t n_qg, int64_t tiles) {
-  const int64_t cus = device_cus();
-  int64_t best = 0;
-  double best_cost = 0.0;
-  const int64_t r0 = (n_qg + cus - 1) / cus;
-  for (int64_t r = r0; r < r0 + 4; ++r) {
-    const int64_t n = r * cus / n_qg;
-    const double cost = (double)r * ((double)tiles / (double)n + (double)kRoundTiles);
-    if (best == 0 || cost < best_cost) {
-      best = n;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
-
 template <typename T, int KS>
 static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   if constexpr (4 * 32 * KS * 16 * T::bytes + kDocTableBytes > 64 * 1024) {
@@ -2228,7 +2089,7 @@ static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   // in the work measure).
   const int64_t w_all = a.total_d + (int64_t)kDocWork * a.nb;
   const int64_t per_table = (int64_t)kDocWork * (kMaxDocsPerGroup - 1);
-  int64_t n_dc = chunks_for_rounds(a.n_qg, w_all / kTileRows);
+  int64_t n_dc = chunks_for_rounds(a.n_qg, w_all / kTileRows, device_cus());
   n_dc = std::max<int64_t>(n_dc, (w_all + per_table - 1) / per_table);
   n_dc = std::max<int64_t>(1, std::min<int64_t>(n_dc, a.nb));
   a.n_dc = (int)n_dc;
@@ -2274,21 +2135,59 @@ static void launch_tiled(const TiledArgs& a, hipStream_t st) {
   }
 }
 
+// Which kernel scores a contrastive batch, and what it needs.
+struct ContrastiveRoute {
+  bool tiled = false;   // contrastive_tiled_kernel
+  bool kloop = false;   // contrastive_kloop_kernel ...
+  bool in_place = false;  // ... which can take the rows as they are
+  bool copy_d = false;    // ... or with the workspace also needs the documents' copy
+  size_t ws = 0;        // ... of this many bytes (0: not worth it)
+};
+
+// A copy of the documents beyond this is not made (the pair kernels read
+// them in place).
+constexpr size_t kMaxDocCopy = (size_t)4 << 30;
+// 16-bit rows that could be used in place have the queries' fragments put in
+// order (one launch more, about 3 us) from this many operations: 7e9 at dim 96
+// ran 33.1 us without and 36.8 us with it, 2e10 at dim 256 101.9 and 83.6 us;
+// fp32, bound by its MFMAs, gained nothing
+constexpr double kFragMinOps = 1e10;
+
+static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int64_t nq,
+                                          int64_t lq, const void* d, int64_t total_d, int64_t nb,
+                                          int64_t dim) {
+  ContrastiveRoute r;
+  const bool ptrs = aligned16(q) && aligned16(d);
+  if (dim == ks_for_dim((int)dim) * kChunk && ptrs) {
+    switch (dtype) {
+      case MAXSIM_BFLOAT16: r.tiled = tiled_supported<BF16>((int)dim, (int)lq); break;
+      case MAXSIM_FLOAT16: r.tiled = tiled_supported<F16>((int)dim, (int)lq); break;
+      default: r.tiled = tiled_supported<F32>((int)dim, (int)lq); break;
+    }
+  }
+  if (r.tiled) return r;
+  const int64_t nblk = (lq + kTileCols - 1) / kTileCols;
+  if (!kloop_supported(dtype, dim, nblk)) return r;
+  r.kloop = true;
+  r.in_place = dim % kChunk == 0 && ptrs;
+  r.copy_d = !(dim % kChunk == 0 && aligned16(d));
+  if (r.in_place && (dtype == MAXSIM_FLOAT32 ||
+                     2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps))
+    return r;
+  r.ws = kloop_workspace_bytes(dtype, nq, nblk, total_d, dim, r.copy_d);
+  if (r.ws > kMaxDocCopy) r.ws = 0;
+  return r;
+}
+
 static int run_contrastive(maxsim_dtype dtype, const void* q, int64_t nq,
                            int64_t lq, const void* d, int64_t total_d,
                            const int32_t* doff, int64_t nb, int64_t dim,
-                           float* scores, int32_t* argmax, hipStream_t st) {
-  const bool vec = (dim == ks_for_dim((int)dim) * kChunk) && aligned16(q) &&
-                   aligned16(d);
-  bool tiled = false;
-  switch (dtype) {
-    case MAXSIM_BFLOAT16: tiled = tiled_supported<BF16>((int)dim, (int)lq); break;
-    case MAXSIM_FLOAT16: tiled = tiled_supported<F16>((int)dim, (int)lq); break;
-    default: tiled = tiled_supported<F32>((int)dim, (int)lq); break;
-  }
-  // The tiled kernel stages whole 16-byte pieces: it needs dim == KS*16 and
-  // aligned rows; other shapes take the pair kernel.
-  if (tiled && vec) {
+                           float* scores, int32_t* argmax, void* workspace,
+                           size_t workspace_bytes, hipStream_t st) {
+  const ContrastiveRoute r = contrastive_route(dtype, q, nq, lq, d, total_d, nb, dim);
+  const bool use_ws =
+      r.kloop && r.ws > 0 && workspace && aligned16(workspace) && workspace_bytes >= r.ws;
+  if (r.tiled || (r.kloop && (r.in_place || use_ws))) {
     TiledArgs a{};
     a.q = q;
     a.d = d;
@@ -2301,6 +2200,11 @@ static int run_contrastive(maxsim_dtype dtype, const void* q, int64_t nq,
     a.nblk = (int)((lq + kTileCols - 1) / kTileCols);
     a.scores = scores;
     a.argmax = argmax;
+    if (r.kloop) {
+      if (use_ws)
+        if (int e = kloop_prepare(dtype, a, r.copy_d, workspace, st)) return e;
+      return launch_contrastive_kloop(dtype, a, st);
+    }
     switch (dtype) {
       case MAXSIM_BFLOAT16: launch_tiled<BF16>(a, st); break;
       case MAXSIM_FLOAT16: launch_tiled<F16>(a, st); break;
@@ -2333,11 +2237,22 @@ using namespace maxsim;
 // ---------------------------------------------------------------------------
 extern "C" {
 
-int maxsim_amd_contrastive_forward_with_argmax(
+size_t maxsim_internal_contrastive_forward_workspace(maxsim_dtype dtype, const void* queries,
+                                                     int64_t num_queries, int64_t Lq,
+                                                     const void* documents, int64_t total_d_tokens,
+                                                     int64_t num_documents, int64_t dim) {
+  if (num_queries <= 0 || num_documents <= 0 || total_d_tokens <= 0 || Lq <= 0 || dim <= 0 ||
+      dim > MAXSIM_AMD_MAX_DIM || Lq > (1 << 20))
+    return 0;
+  return contrastive_route(dtype, queries, num_queries, Lq, documents, total_d_tokens,
+                           num_documents, dim).ws;
+}
+
+int maxsim_internal_contrastive_forward(
     maxsim_dtype dtype, const void* queries, int64_t num_queries, int64_t Lq,
     const void* documents, int64_t total_d_tokens,
     const int32_t* document_offsets, int64_t num_documents, int64_t dim,
-    float* scores, int32_t* argmax, void* stream) {
+    float* scores, int32_t* argmax, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   if (int e = check_dtype(dtype)) return e;
   if (num_queries < 0 || num_documents < 0 || total_d_tokens < 0)
@@ -2351,7 +2266,18 @@ int maxsim_amd_contrastive_forward_with_argmax(
     return fail(MAXSIM_ERR_UNSUPPORTED, "problem too large");
   return run_contrastive(dtype, queries, num_queries, Lq, documents,
                          total_d_tokens, document_offsets, num_documents, dim,
-                         scores, argmax, static_cast<hipStream_t>(stream));
+                         scores, argmax, workspace, workspace_bytes,
+                         static_cast<hipStream_t>(stream));
+}
+
+int maxsim_amd_contrastive_forward_with_argmax(
+    maxsim_dtype dtype, const void* queries, int64_t num_queries, int64_t Lq,
+    const void* documents, int64_t total_d_tokens,
+    const int32_t* document_offsets, int64_t num_documents, int64_t dim,
+    float* scores, int32_t* argmax, void* stream) {
+  return maxsim_internal_contrastive_forward(dtype, queries, num_queries, Lq, documents,
+                                             total_d_tokens, document_offsets, num_documents, dim,
+                                             scores, argmax, nullptr, 0, stream);
 }
 
 int maxsim_amd_contrastive_forward(maxsim_dtype dtype, const void* queries,

@@ -16,7 +16,7 @@
 #include <tuple>
 #include <vector>
 
-#include "../../include/maxsim_amd.h"
+#include "maxsim_internal.h"
 
 namespace {
 
@@ -395,6 +395,21 @@ Contrastive prep_contrastive(Tensor queries, Tensor documents, Tensor document_o
   return c;
 }
 
+// The forward with the workspace its kernel can use, if any (from torch's
+// allocator, on the current stream like the launches that use it).
+void run_contrastive_forward(const Contrastive& c, int64_t nq, int64_t lq, int64_t nb,
+                             const Tensor& scores, int32_t* argmax) {
+  const maxsim_dtype dt = to_dtype(c.q);
+  const size_t bytes = maxsim_internal_contrastive_forward_workspace(
+      dt, c.q.data_ptr(), nq, lq, c.d.data_ptr(), c.d.size(0), nb, c.q.size(2));
+  Tensor ws;
+  if (bytes > 0) ws = at::empty({(int64_t)bytes}, c.q.options().dtype(at::kByte));
+  check_status(maxsim_internal_contrastive_forward(
+      dt, c.q.data_ptr(), nq, lq, c.d.data_ptr(), c.d.size(0), c.off.data_ptr<int32_t>(), nb,
+      c.q.size(2), scores.data_ptr<float>(), argmax, bytes > 0 ? ws.data_ptr() : nullptr, bytes,
+      current_stream(c.q)));
+}
+
 Tensor maxsim_contrastive_forward(Tensor queries, Tensor documents,
                                   Tensor document_offsets) {
   Contrastive c = prep_contrastive(queries, documents, document_offsets);
@@ -402,10 +417,7 @@ Tensor maxsim_contrastive_forward(Tensor queries, Tensor documents,
   Tensor scores = at::empty({Nq, Nb}, f32_opts(c.q));
   if (Nq * Nb == 0) return scores;
   c10::hip::HIPGuardMasqueradingAsCUDA guard(c.q.device());
-  check_status(maxsim_amd_contrastive_forward(
-      to_dtype(c.q), c.q.data_ptr(), Nq, Lq, c.d.data_ptr(), c.d.size(0),
-      c.off.data_ptr<int32_t>(), Nb, c.q.size(2), scores.data_ptr<float>(),
-      current_stream(c.q)));
+  run_contrastive_forward(c, Nq, Lq, Nb, scores, nullptr);
   return scores;
 }
 
@@ -417,10 +429,7 @@ std::tuple<Tensor, Tensor> maxsim_contrastive_forward_with_argmax(
   Tensor argmax = at::empty({Nq, Nb, Lq}, i32_opts(c.q));
   if (Nq * Nb == 0) return {scores, argmax};
   c10::hip::HIPGuardMasqueradingAsCUDA guard(c.q.device());
-  check_status(maxsim_amd_contrastive_forward_with_argmax(
-      to_dtype(c.q), c.q.data_ptr(), Nq, Lq, c.d.data_ptr(), c.d.size(0),
-      c.off.data_ptr<int32_t>(), Nb, c.q.size(2), scores.data_ptr<float>(),
-      argmax.data_ptr<int32_t>(), current_stream(c.q)));
+  run_contrastive_forward(c, Nq, Lq, Nb, scores, argmax.data_ptr<int32_t>());
   return {scores, argmax};
 }
 
