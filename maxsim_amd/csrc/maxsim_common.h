@@ -57,22 +57,58 @@ __device__ __forceinline__ Frag<T> zero_frag() {
   return f;
 }
 
-// Load 8 elements [k0, k0+8) of a row.  `vec` means the row pointer plus k0
-// is 16-byte aligned and k0 + 8 <= dim; otherwise elements at k >= dim read
-// as zero and the load is element-wise.
+// 16 bytes from an address that is only a multiple of the element size (the
+// compiler knows what the target's loads need).
+template <typename S>
+__device__ __forceinline__ uint4 load16_any(const S* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+
+// v without its first n bytes (0 <= n), zeros behind; n may differ by lane.
+__device__ __forceinline__ uint4 drop_bytes(uint4 v, int n) {
+  uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+  const int b = 8 * (n & 7);
+  const uint64_t lo1 = n >= 8 ? hi : lo, hi1 = n >= 8 ? 0 : hi;
+  const uint64_t up = (hi1 << 1) << (63 - b);  // hi1 << (64 - b), 0 for b = 0
+  lo = n >= 16 ? 0 : (lo1 >> b) | up;
+  hi = n >= 16 ? 0 : hi1 >> b;
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+// Elements [k0, k0 + 8) of a row that starts anywhere, those at k >= dim read
+// as zero, in two parts for dim >= 8: the loads, whole and unconditional (a
+// fragment at the row's end reads its last elements instead), and, where the
+// data is used, the move into place.  The second is needed only where k0 + 8
+// > dim; keeping it away from the loads lets a tile's loads stay in flight.
 template <typename T>
-__device__ __forceinline__ Frag<T> load_frag(const typename T::storage* row,
-                                             int k0, int dim, bool vec) {
+__device__ __forceinline__ Frag<T> load_frag_any(const typename T::storage* row, int k0,
+                                                 int dim) {
   Frag<T> f;
-  if (vec) {
-    if constexpr (T::bytes == 2) {
-      f.v = *reinterpret_cast<const uint4*>(row + k0);
-    } else {
-      f.lo = *reinterpret_cast<const uint4*>(row + k0);
-      f.hi = *reinterpret_cast<const uint4*>(row + k0 + 4);
-    }
-    return f;
+  if constexpr (T::bytes == 2) {
+    f.v = load16_any(row + min(k0, dim - 8));
+  } else {
+    f.lo = load16_any(row + min(k0, dim - 4));
+    f.hi = load16_any(row + min(k0 + 4, dim - 4));
   }
+  return f;
+}
+template <typename T>
+__device__ __forceinline__ void place_frag(Frag<T>& f, int k0, int dim) {
+  if constexpr (T::bytes == 2) {
+    f.v = drop_bytes(f.v, 2 * max(k0 - (dim - 8), 0));
+  } else {
+    f.lo = drop_bytes(f.lo, 4 * max(k0 - (dim - 4), 0));
+    f.hi = drop_bytes(f.hi, 4 * max(k0 + 4 - (dim - 4), 0));
+  }
+}
+
+// The same element by element, for rows of any length.
+template <typename T>
+__device__ __forceinline__ Frag<T> load_frag_short(const typename T::storage* row, int k0,
+                                                   int dim) {
+  Frag<T> f;
   if constexpr (T::bytes == 2) {
     uint32_t w[4];
 #pragma unroll
@@ -93,6 +129,62 @@ __device__ __forceinline__ Frag<T> load_frag(const typename T::storage* row,
                       __float_as_uint(x[6]), __float_as_uint(x[7]));
   }
   return f;
+}
+
+// Load 8 elements [k0, k0+8) of a row.  `vec` means the row pointer plus k0
+// is 16-byte aligned and k0 + 8 <= dim; otherwise the row may start anywhere
+// and elements at k >= dim read as zero.
+template <typename T>
+__device__ __forceinline__ Frag<T> load_frag(const typename T::storage* row,
+                                             int k0, int dim, bool vec) {
+  Frag<T> f;
+  if (vec) {
+    if constexpr (T::bytes == 2) {
+      f.v = *reinterpret_cast<const uint4*>(row + k0);
+    } else {
+      f.lo = *reinterpret_cast<const uint4*>(row + k0);
+      f.hi = *reinterpret_cast<const uint4*>(row + k0 + 4);
+    }
+    return f;
+  }
+  if (dim < 8) return load_frag_short<T>(row, k0, dim);
+  f = load_frag_any<T>(row, k0, dim);
+  if (k0 + 8 > dim) place_frag<T>(f, k0, dim);
+  return f;
+}
+
+// A row's KS chunks (16 elements each, this lane's halves at 8 * h) for the
+// kernels that hold a whole row, by a constant of the launch: aligned whole
+// fragments; rows of at least 8 elements that start anywhere; shorter ones,
+// element by element.  Chunks past the embedding dimension are neither loaded
+// nor (mma_chunks) multiplied.  (Its own constant for the short rows: their
+// loads' many branches would spill scalar registers in every kernel.)  Rows
+// of widths such as 96, 100 or 300 were read element by element before:
+// packed bf16 dim 96, 777 pairs 66 -> 13.5 us; padded fp16 dim 300, 28k pairs
+// 2658 -> 685 us; padded bf16 dim 96, 6400 pairs of up to 300 rows 278 -> 52 us
+// (same bits).
+enum RowLoad : int { kRowShort = 0, kRowVec = 1, kRowAny = 2 };
+template <typename T, int KS, int LOAD>
+__device__ __forceinline__ void load_row(const typename T::storage* row, int h, int dim,
+                                         Frag<T> (&f)[KS]) {
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    if constexpr (LOAD == kRowVec)
+      f[s] = load_frag<T>(row, kChunk * s + 8 * h, dim, true);
+    else if constexpr (LOAD == kRowShort)
+      f[s] = load_frag_short<T>(row, kChunk * s + 8 * h, dim);
+    else if (kChunk * s < dim)
+      f[s] = load_frag_any<T>(row, kChunk * s + 8 * h, dim);
+  }
+}
+// The fragments of load_row in place (needed once per loaded row).
+template <typename T, int KS, int LOAD>
+__device__ __forceinline__ void place_row(Frag<T> (&f)[KS], int h, int dim) {
+  if constexpr (LOAD == kRowAny) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      if (kChunk * s < dim && kChunk * s + kChunk > dim) place_frag<T>(f[s], kChunk * s + 8 * h, dim);
+  }
 }
 
 // acc += A(32 rows x 16 k) * B(16 k x 32 tokens) for one K-chunk.
@@ -118,6 +210,15 @@ __device__ __forceinline__ void mma_chunk(const Frag<F32>& a,
   for (int e = 0; e < 8; ++e)
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(
         __uint_as_float(av[e]), __uint_as_float(bv[e]), acc, 0, 0, 0);
+}
+
+// acc += the product of two rows' chunks (load_row), in order.
+template <typename T, int KS, int LOAD>
+__device__ __forceinline__ void mma_chunks(const Frag<T> (&a)[KS], const Frag<T> (&b)[KS], int dim,
+                                           f32x16& acc) {
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    if (LOAD != kRowAny || kChunk * s < dim) mma_chunk(a[s], b[s], acc);
 }
 
 // Row (within the 32-row tile) held by accumulator register r of lane-half h.

@@ -131,13 +131,11 @@ __device__ __forceinline__ void write_invalid_pair(const FwdArgs& a, int64_t p,
 // QB query blocks (32 tokens each) are held in registers; queries longer than
 // 32*QB tokens are processed QB blocks at a time, re-streaming the document.
 // ---------------------------------------------------------------------------
-// VEC (rows are whole 16-byte fragments, 16-byte aligned) is a template
-// parameter: as a runtime flag, both load paths were compiled into the tile
-// loop, and the element-wise one's bounds checks drove the kernel into
-// scalar-register spills.
-template <typename T, int KS, int QB, bool ARGMAX, bool VEC>
+// How rows are loaded is a template parameter: as a runtime flag, both load
+// paths were compiled into the tile loop, and the general one's bounds checks
+// drove the kernel into scalar-register spills.
+template <typename T, int KS, int QB, bool ARGMAX, int LOAD>
 __global__ __launch_bounds__(256) void pair_kernel(FwdArgs a, int ppw) {
-  constexpr bool vec = VEC;
   using S = typename T::storage;
   const int lane = threadIdx.x & 63;
   const int c = lane & 31;
@@ -162,9 +160,7 @@ __global__ __launch_bounds__(256) void pair_kernel(FwdArgs a, int ppw) {
   // first tile already in flight (queries that change still load here).
   auto load_tile = [&](const Pair& q_pr, int t, Frag<T> (&f)[KS]) __attribute__((always_inline)) {
     const int r = min(t * kTileRows + c, q_pr.ld - 1);
-    const S* row = D + (q_pr.d_row0 + r) * (int64_t)dim;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) f[s] = load_frag<T>(row, kChunk * s + 8 * h, dim, vec);
+    load_row<T, KS, LOAD>(D + (q_pr.d_row0 + r) * (int64_t)dim, h, dim, f);
   };
   Pair pr = resolve_pair(a, p_begin);
   Frag<T> df[KS];
@@ -189,10 +185,8 @@ __global__ __launch_bounds__(256) void pair_kernel(FwdArgs a, int ppw) {
         for (int qb = 0; qb < QB; ++qb) {
           if (qb >= nact) break;
           const int tok = min((g0 + qb) * kTileCols + c, pr.lq - 1);
-          const S* row = Q + (pr.q_row0 + tok) * (int64_t)dim;
-#pragma unroll
-          for (int s = 0; s < KS; ++s)
-            qf[qb][s] = load_frag<T>(row, kChunk * s + 8 * h, dim, vec);
+          load_row<T, KS, LOAD>(Q + (pr.q_row0 + tok) * (int64_t)dim, h, dim, qf[qb]);
+          place_row<T, KS, LOAD>(qf[qb], h, dim);
         }
         loaded_q = pr.q_row0;
         loaded_lq = pr.lq;
@@ -223,12 +217,12 @@ __global__ __launch_bounds__(256) void pair_kernel(FwdArgs a, int ppw) {
             load_tile(nx, 0, nf);
           // rows past the document end were loaded as copies of its last row
           // and cannot win (see tile_update), so no masking is needed
+          place_row<T, KS, LOAD>(df, h, dim);
           f32x16 acc[NA];
 #pragma unroll
           for (int qb = 0; qb < NA; ++qb) {
             acc[qb] = f32x16{};
-#pragma unroll
-            for (int s = 0; s < KS; ++s) mma_chunk(df[s], qf[qb][s], acc[qb]);
+            mma_chunks<T, KS, LOAD>(df, qf[qb], dim, acc[qb]);
           }
 #pragma unroll
           for (int qb = 0; qb < NA; ++qb)
@@ -279,7 +273,7 @@ __global__ __launch_bounds__(256) void pair_kernel(FwdArgs a, int ppw) {
 // ---------------------------------------------------------------------------
 constexpr int kSplitWaves = 4;
 
-template <typename T, int KS, bool ARGMAX, bool VEC>
+template <typename T, int KS, bool ARGMAX, int LOAD>
 __global__ __launch_bounds__(kSplitWaves * 64) void pair_split_kernel(FwdArgs a) {
   using S = typename T::storage;
   __shared__ float sm[kSplitWaves][kTileCols];
@@ -302,31 +296,28 @@ __global__ __launch_bounds__(kSplitWaves * 64) void pair_split_kernel(FwdArgs a)
   const int ntiles = (pr.ld + kTileRows - 1) / kTileRows;
   auto load_tile = [&](int t, Frag<T> (&f)[KS]) __attribute__((always_inline)) {
     const int r = min(t * kTileRows + c, pr.ld - 1);
-    const S* row = D + (pr.d_row0 + r) * (int64_t)dim;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) f[s] = load_frag<T>(row, kChunk * s + 8 * h, dim, VEC);
+    load_row<T, KS, LOAD>(D + (pr.d_row0 + r) * (int64_t)dim, h, dim, f);
   };
   float score = 0.0f;
   for (int blk = 0; blk < nblk; ++blk) {
     Frag<T> qf[KS];
     {
       const int tok = min(blk * kTileCols + c, pr.lq - 1);
-      const S* row = Q + (pr.q_row0 + tok) * (int64_t)dim;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) qf[s] = load_frag<T>(row, kChunk * s + 8 * h, dim, VEC);
+      load_row<T, KS, LOAD>(Q + (pr.q_row0 + tok) * (int64_t)dim, h, dim, qf);
     }
     float m = -__builtin_inff();
     int am = 0;
     // this wave's tiles, the next one's fragments loading while one is scored
     Frag<T> df[KS];
     if (w < ntiles) load_tile(w, df);
+    place_row<T, KS, LOAD>(qf, h, dim);
     for (int t = w; t < ntiles; t += kSplitWaves) {
       Frag<T> nf[KS];
       const bool more = t + kSplitWaves < ntiles;
       if (more) load_tile(t + kSplitWaves, nf);
+      place_row<T, KS, LOAD>(df, h, dim);
       f32x16 acc = f32x16{};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) mma_chunk(df[s], qf[s], acc);
+      mma_chunks<T, KS, LOAD>(df, qf, dim, acc);
       tile_update<ARGMAX>(acc, m, am, t * kTileRows + 4 * h);
       if (more) {
 #pragma unroll
@@ -410,13 +401,22 @@ __global__ __launch_bounds__(256) void wide_pair_kernel(FwdArgs a) {
 #pragma unroll
         for (int u = 0; u < kWideBatch; ++u) {
           const int k0 = kChunk * (s0 + u) + 8 * h;
-          const bool in = s0 + u < ks;
-          fa[u] = in ? load_frag<T>(drow, k0, dim, VEC) : zero_frag<T>();
-          fb[u] = in ? load_frag<T>(qrow, k0, dim, VEC) : zero_frag<T>();
+          if (s0 + u < ks) {
+            fa[u] = VEC ? load_frag<T>(drow, k0, dim, true) : load_frag_any<T>(drow, k0, dim);
+            fb[u] = VEC ? load_frag<T>(qrow, k0, dim, true) : load_frag_any<T>(qrow, k0, dim);
+          }
         }
 #pragma unroll
-        for (int u = 0; u < kWideBatch; ++u)
-          if (s0 + u < ks) mma_chunk(fa[u], fb[u], acc);
+        for (int u = 0; u < kWideBatch; ++u) {
+          if (s0 + u < ks) {
+            const int k0 = kChunk * (s0 + u) + 8 * h;
+            if (!VEC && kChunk * (s0 + u + 1) > dim) {
+              place_frag<T>(fa[u], k0, dim);
+              place_frag<T>(fb[u], k0, dim);
+            }
+            mma_chunk(fa[u], fb[u], acc);
+          }
+        }
       }
       tile_update<ARGMAX>(acc, m, am, t * kTileRows + 4 * h);
     }
@@ -1803,17 +1803,20 @@ static bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
 
+template <typename T, int KS, int QB, int LOAD>
+static void launch_pair_load(const FwdArgs& a, int ppw, dim3 grid, hipStream_t st) {
+  hipLaunchKernelGGL((a.argmax ? pair_kernel<T, KS, QB, true, LOAD>
+                               : pair_kernel<T, KS, QB, false, LOAD>),
+                     grid, dim3(256), 0, st, a, ppw);
+}
+
 template <typename T, int KS, int QB>
 static void launch_pair_qb(const FwdArgs& a, int ppw, bool vec, dim3 grid,
                            hipStream_t st) {
-  if (a.argmax && vec)
-    hipLaunchKernelGGL((pair_kernel<T, KS, QB, true, true>), grid, dim3(256), 0, st, a, ppw);
-  else if (a.argmax)
-    hipLaunchKernelGGL((pair_kernel<T, KS, QB, true, false>), grid, dim3(256), 0, st, a, ppw);
-  else if (vec)
-    hipLaunchKernelGGL((pair_kernel<T, KS, QB, false, true>), grid, dim3(256), 0, st, a, ppw);
-  else
-    hipLaunchKernelGGL((pair_kernel<T, KS, QB, false, false>), grid, dim3(256), 0, st, a, ppw);
+  if (vec) return launch_pair_load<T, KS, QB, kRowVec>(a, ppw, grid, st);
+  if constexpr (KS == 2)
+    if (a.dim < 8) return launch_pair_load<T, KS, QB, kRowShort>(a, ppw, grid, st);
+  launch_pair_load<T, KS, QB, kRowAny>(a, ppw, grid, st);
 }
 
 template <typename T, int KS>
@@ -1840,18 +1843,19 @@ static void launch_pair(const FwdArgs& a, int max_lq, int ppw, bool vec,
   }
 }
 
+template <typename T, int KS, int LOAD>
+static void launch_split_load(const FwdArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((a.argmax ? pair_split_kernel<T, KS, true, LOAD>
+                               : pair_split_kernel<T, KS, false, LOAD>),
+                     dim3((unsigned)a.npairs), dim3(kSplitWaves * 64), 0, st, a);
+}
+
 template <typename T, int KS>
 static void launch_split_ks(const FwdArgs& a, bool vec, hipStream_t st) {
-  const dim3 grid((unsigned)a.npairs);
-  const dim3 block(kSplitWaves * 64);
-  if (a.argmax && vec)
-    hipLaunchKernelGGL((pair_split_kernel<T, KS, true, true>), grid, block, 0, st, a);
-  else if (a.argmax)
-    hipLaunchKernelGGL((pair_split_kernel<T, KS, true, false>), grid, block, 0, st, a);
-  else if (vec)
-    hipLaunchKernelGGL((pair_split_kernel<T, KS, false, true>), grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL((pair_split_kernel<T, KS, false, false>), grid, block, 0, st, a);
+  if (vec) return launch_split_load<T, KS, kRowVec>(a, st);
+  if constexpr (KS == 2)
+    if (a.dim < 8) return launch_split_load<T, KS, kRowShort>(a, st);
+  launch_split_load<T, KS, kRowAny>(a, st);
 }
 
 template <typename T>

@@ -1,0 +1,56 @@
+"""Padded and packed forwards over embedding widths that are not whole aligned
+fragments: every remainder of a row's last 8 elements, rows on any element
+boundary, the pair kernels of few and of many pairs, wide rows."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import maxsim_amd
+from maxsim_amd._ops import ops
+from oracle import maxsim_oracle as oracle
+
+from ._helpers import (DTYPES, SCORE_TOL, assert_close, check_argmax, make_packed, make_padded,
+                       np64, npi)
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [1, 7, 8, 9, 15, 16, 17, 26, 35, 44, 61, 96, 100, 118, 127, 143, 201, 255, 300, 301]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("dim", WIDTHS)
+def test_padded_forward_row_widths(dim, dtype):
+    q, d, ql, dl = make_padded(3, 5, 35, 40, dim, dtype, seed=dim)
+    s, a = maxsim_amd.score_candidates_padded_with_argmax(q, d, ql, dl)
+    qn, dn = np64(q), np64(d)
+    s_ref, a_ref = oracle.padded_forward(qn, dn, npi(ql), npi(dl))
+    # |q||d| grows like sqrt(dim): the absolute floor with it
+    tol = dict(SCORE_TOL[dtype], atol=SCORE_TOL[dtype]["atol"] * max(1.0, dim / 64))
+    assert_close(s, s_ref, **tol)
+    check_argmax(npi(a), a_ref, lambda i: qn[i[0], i[2]], lambda i, j: dn[i[0], i[1], j])
+    # rows that start one element off give the same bits
+    qs, ds = (torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view_as(t).copy_(t)
+              for t in (q, d))
+    s2, a2 = maxsim_amd.score_candidates_padded_with_argmax(qs, ds, ql, dl)
+    assert torch.equal(s, s2) and torch.equal(a, a2)
+
+
+@pytest.mark.parametrize("dim,dtype", [(20, torch.bfloat16), (96, torch.float16),
+                                       (100, torch.float32), (201, torch.bfloat16),
+                                       (300, torch.float16)])
+def test_packed_forward_row_widths_many_pairs(dim, dtype):
+    """1100 pairs (a wave per pair) against the same pairs in small batches (a
+    workgroup per pair), bit for bit, and the last row of the last document at
+    the end of its allocation."""
+    args = make_packed(20, 60, 1100, dim, (1, 40), (1, 70), dtype, seed=dim)
+    q, qo, d, do, qi, di = args
+    s, a = ops.maxsim_packed_forward_with_argmax(q, qo, d, do, qi, di, 40)
+    for lo in (0, 700):
+        s2, a2 = ops.maxsim_packed_forward_with_argmax(q, qo, d, do, qi[lo:lo + 400].contiguous(),
+                                                       di[lo:lo + 400].contiguous(), 40)
+        assert torch.equal(s[lo:lo + 400], s2) and torch.equal(a[lo:lo + 400], a2)
+    s_ref, _ = oracle.packed_forward(np64(q), npi(qo), np64(d), npi(do), npi(qi), npi(di), 40)
+    tol = dict(SCORE_TOL[dtype], atol=SCORE_TOL[dtype]["atol"] * max(1.0, dim / 64))
+    assert_close(s, s_ref, **tol)
