@@ -84,9 +84,9 @@ def set_host_checks(enabled: bool) -> bool:
     default) or off, process-wide; returns the previous setting.  The
     environment variable ``MAXSIM_AMD_HOST_CHECKS=0`` sets it off at import.
 
-    On, every call copies its offsets / ids / lengths to the host and raises
+    On, every call checks its offsets / ids / lengths on the device and raises
     the reference's errors for invalid values, which makes the host wait for
-    that copy once per call (overlapped with the kernels, but a wait).
+    that check once per call (overlapped with the kernels, but a wait).
 
     Off, a call on device tensors never waits for the device: only the checks
     that need no device data run (shapes, dtypes, devices), and the kernels'
@@ -167,36 +167,16 @@ def _to_host(*tensors: torch.Tensor) -> list[np.ndarray]:
     return out
 
 
-_COPY_STREAMS: dict = {}
-
-
-def _host_copies_async(*tensors: torch.Tensor):
-    """Queue device->host copies of small int tensors into pinned memory on a
-    side stream (default priority, one per device) and return the host
-    tensors and an event that marks their completion.
-
-    The side stream first waits for the work already queued on the current
-    stream, so the copies see every earlier write of their sources.  Kernels
-    queued on the current stream afterwards do not wait for the copies: the
-    validation copies stay off the compute stream.  Used where the kernels
-    run many small workgroups (padded, packed), so the copies' blit kernels
-    find a free CU at once."""
-    device = tensors[0].device
-    cur = torch.cuda.current_stream(device)
-    side = _COPY_STREAMS.get(device.index)
-    if side is None:
-        side = _COPY_STREAMS[device.index] = torch.cuda.Stream(device)
-    side.wait_stream(cur)
-    hosts = []
-    with torch.cuda.stream(side):
-        for t in tensors:
-            flat = t.detach().reshape(-1)
-            host = torch.empty(flat.shape, dtype=flat.dtype, pin_memory=True)
-            host.copy_(flat, non_blocking=True)
-            hosts.append(host)
-        done = torch.cuda.Event()
-        done.record(side)
-    return hosts, done
+def _run_checked(status, like, launch):
+    """``launch()`` while the layout check ``status`` (queued on the current
+    stream ahead of it) runs; returns its result and what the check found:
+    the longest segment of its first array, or -1 for a bad value.  Waits for
+    the check also when ``launch`` raises: the check writes ``status``."""
+    try:
+        result = launch()
+    finally:
+        found = ops.maxsim_check_wait(status, like)
+    return result, found
 
 
 def _check_lengths(values: np.ndarray, max_len: int, name: str) -> None:
@@ -242,37 +222,35 @@ def _check_padded_meta(queries, documents, query_lengths, doc_lengths):
     return B, C, Lq, Ld, D
 
 
-# The _checked_* wrappers are host code (pinned copies, events, numpy checks);
-# torch.compile runs them eagerly at a graph break, as it does the
+# The _checked_* wrappers are host code (a pinned buffer, a wait); torch.compile
+# runs them eagerly at a graph break, as it does the
 # reference's host-side checks.  The operators they launch have fake
 # implementations and trace on their own.
 @torch.compiler.disable
 def _checked_padded(queries, documents, query_lengths, doc_lengths, launch):
     """Validate a padded call and return ``launch(B, C, Lq, Ld)``.
 
-    The lengths travel to pinned host memory by asynchronous copies on a side
-    stream (:func:`_host_copies_async`), ``launch`` queues the kernels, and
-    only then does the host wait for the copies and check the values, with the same errors
-    as a check made before the launch.  The padded kernels are safe with any
-    lengths (a candidate with a length outside ``(0, Ld]`` or a query length
-    outside ``(0, Lq]`` gives a NaN score, nothing is read out of range), so
-    work queued before a failing check is harmless and its result is
-    dropped."""
+    A small kernel checks the lengths on the device and writes its verdict
+    into pinned host memory; ``launch`` queues the kernels behind it, and only
+    then does the host wait for the verdict.  A bad one copies the lengths to
+    the host for the reference's errors.  The padded kernels are safe with
+    any lengths (a candidate with a length outside ``(0, Ld]`` or a query
+    length outside ``(0, Lq]`` gives a NaN score, nothing is read out of
+    range), so work queued before a failing check is harmless and its result
+    is dropped."""
     B, C, Lq, Ld, _ = _check_padded_meta(queries, documents, query_lengths, doc_lengths)
     if not _HOST_CHECKS and query_lengths.is_cuda:
         return launch(B, C, Lq, Ld)
-    if not query_lengths.is_cuda:  # host tensors: check first (the operators reject them anyway)
-        qlen, dlen = _to_host(query_lengths, doc_lengths)
-        _check_lengths(qlen, Lq, "query_lengths")
-        _check_lengths(dlen, Ld, "doc_lengths")
-        return launch(B, C, Lq, Ld)
-    hosts, copied = _host_copies_async(query_lengths, doc_lengths)
-    result = launch(B, C, Lq, Ld)
-    copied.synchronize()
-    qlen, dlen = (h.numpy().astype(np.int64) for h in hosts)
+    if query_lengths.is_cuda:
+        status = ops.maxsim_check_padded(query_lengths, doc_lengths, Lq, Ld)
+        result, found = _run_checked(status, query_lengths, lambda: launch(B, C, Lq, Ld))
+        if found >= 0:
+            return result
+    # a bad length, or host tensors (the operators reject them anyway)
+    qlen, dlen = _to_host(query_lengths, doc_lengths)
     _check_lengths(qlen, Lq, "query_lengths")
     _check_lengths(dlen, Ld, "doc_lengths")
-    return result
+    return launch(B, C, Lq, Ld)
 
 
 def _check_pair_ids(pair_query_ids, pair_document_ids) -> None:
@@ -339,56 +317,49 @@ def _checked_packed(queries, query_offsets, documents, document_offsets,
                     shape_needs_max=True):
     """Validate a packed call and return ``launch(max_q_len)``.
 
-    The offsets and ids travel to pinned host memory by asynchronous copies
-    on a side stream (:func:`_host_copies_async`), ``launch`` queues the
-    kernels, and only then does the host wait for the copies and run the
-    reference's checks with its errors.  The packed kernels are safe with
-    any offsets and ids (an invalid pair gives a NaN score, nothing is read
-    out of range), so work queued before a failing check is harmless and its
-    result is dropped.
+    A small kernel checks the offsets and ids on the device and writes its
+    verdict and the longest query into pinned host memory; ``launch`` queues
+    the kernels behind it, and only then does the host wait for the verdict.
+    A bad one copies the arrays to the host for the reference's errors.  The
+    packed kernels are safe with any offsets and ids (an invalid pair gives a
+    NaN score, nothing is read out of range), so work queued before a failing
+    check is harmless and its result is dropped.
 
     Without ``max_q_len`` the launch needs a bound of the query lengths.  A
     score-only call (``shape_needs_max=False``) uses the number of query
     rows, which bounds every valid segment and gives the same scores.  Where
-    the argmax shape is the longest query, that length is computed on the
-    device and read back as one integer; offsets that cannot be well formed
-    take the synchronous checks first."""
-    if not query_offsets.is_cuda:  # host tensors: check first (the operators reject them)
-        return launch(_resolve_max_q_len(max_q_len, _packed_layout(
+    the argmax shape is the longest query, the check's finding is waited for
+    before the launch."""
+    total_q = int(queries.shape[0])
+
+    def on_host():
+        return _resolve_max_q_len(max_q_len, _packed_layout(
             queries, query_offsets, documents, document_offsets,
-            pair_query_ids, pair_document_ids)))
+            pair_query_ids, pair_document_ids))
+
+    if not query_offsets.is_cuda:  # host tensors: check first (the operators reject them)
+        return launch(on_host())
     if max_q_len is not None and max_q_len <= 0:
         raise ValueError(f"max_q_len must be > 0; got {max_q_len}")
     if not _HOST_CHECKS:
         if max_q_len is not None:
             return launch(int(max_q_len))
         if not shape_needs_max:
-            return launch(max(int(queries.shape[0]), 1))
-        mql = _device_max_segment(query_offsets, int(queries.shape[0]))
+            return launch(max(total_q, 1))
+        mql = _device_max_segment(query_offsets, total_q)
         # offsets that cannot be well formed: every pair is invalid anyway
         return launch(mql if mql is not None else 1)
-    # queued before the read-back below, so that only the launch sits
-    # between the host's wait for the longest query and the kernels
-    hosts, copied = _host_copies_async(query_offsets, document_offsets, pair_query_ids,
-                                       pair_document_ids)
+    status = ops.maxsim_check_packed(query_offsets, document_offsets, pair_query_ids,
+                                     pair_document_ids, total_q, int(documents.shape[0]))
+    if max_q_len is None and shape_needs_max:
+        found = ops.maxsim_check_wait(status, query_offsets)
+        return launch(found if found >= 0 else on_host())
+    mql = int(max_q_len) if max_q_len is not None else max(total_q, 1)
+    result, found = _run_checked(status, query_offsets, lambda: launch(mql))
+    if found < 0:
+        return launch(on_host())
     if max_q_len is not None:
-        mql = int(max_q_len)
-    elif not shape_needs_max:
-        mql = max(int(queries.shape[0]), 1)
-    else:
-        mql = _device_max_segment(query_offsets, int(queries.shape[0]))
-        if mql is None:
-            return launch(_packed_layout(queries, query_offsets, documents, document_offsets,
-                                         pair_query_ids, pair_document_ids))
-    result = launch(mql)
-    copied.synchronize()
-    qoff, doff, qids, dids = (h.numpy().astype(np.int64) for h in hosts)
-    max_q = _check_csr(qoff, queries.shape[0], "query_offsets")
-    _check_csr(doff, documents.shape[0], "document_offsets")
-    _check_ids(qids, qoff.size - 1, "pair_query_ids")
-    _check_ids(dids, doff.size - 1, "pair_document_ids")
-    if max_q_len is not None:
-        _resolve_max_q_len(max_q_len, max_q)
+        _resolve_max_q_len(max_q_len, found)
     return result
 
 
@@ -759,46 +730,30 @@ def _check_targets(t: np.ndarray, nb: int) -> None:
 def _checked_contrastive(queries, documents, document_offsets, launch, targets=None):
     """Validate a contrastive call and return ``launch()``.
 
-    The offsets (and the cross-entropy targets, when given) travel to pinned
-    host memory by asynchronous copies queued ahead of the kernels, and
-    ``launch()`` queues the kernels before the host waits for those copies,
-    so the GPU is never idle while the host checks them.  Invalid offsets or
-    targets raise the same errors as before; the kernels already queued are
-    safe with any offsets and targets (documents with an invalid range give
-    NaN, a target outside ``[0, Nb)`` a NaN loss, nothing is read out of
-    range) and their results are dropped."""
+    A small kernel checks the offsets (and the cross-entropy targets, when
+    given) on the device and writes its verdict into pinned host memory;
+    ``launch()`` queues the kernels behind it before the host waits for the
+    verdict, so the GPU is never idle meanwhile.  A bad one copies them to the
+    host for the reference's errors; the kernels already queued are safe with
+    any offsets and targets (documents with an invalid range give NaN, a
+    target outside ``[0, Nb)`` a NaN loss, nothing is read out of range) and
+    their results are dropped."""
     _check_contrastive(queries, documents, document_offsets)
-    flat = document_offsets.detach().reshape(-1)
-    nb = flat.numel() - 1
+    flat = document_offsets.detach()
     if not _HOST_CHECKS and flat.is_cuda:
         if documents.shape[0] == 0:
             raise ValueError("documents must not be empty (document_offsets has >= 1 document)")
         return launch()
-    if not flat.is_cuda:  # host tensors: check first (the operators reject them anyway)
-        _check_offsets(flat.numpy().astype(np.int64), documents.shape[0])
-        if targets is not None:
-            _check_targets(_to_host(targets)[0], nb)
-        return launch()
-    # The copy stays on the current stream: a small copy runs as a blit
-    # kernel, and on a side stream it would wait for a free CU until the
-    # contrastive forward (one large workgroup per CU) ends, keeping the host
-    # from queueing the next launches in time.  In the stream it costs a few
-    # microseconds between the previous step's work and the forward.
-    host = torch.empty(flat.shape, dtype=flat.dtype, pin_memory=True)
-    host.copy_(flat, non_blocking=True)
-    host_t = None
+    if flat.is_cuda:
+        status = ops.maxsim_check_contrastive(flat, int(documents.shape[0]), targets)
+        result, found = _run_checked(status, flat, launch)
+        if found >= 0:
+            return result
+    # a bad value, or host tensors (the operators reject them anyway)
+    _check_offsets(_to_host(flat)[0], documents.shape[0])
     if targets is not None:
-        tflat = targets.detach().reshape(-1)
-        host_t = torch.empty(tflat.shape, dtype=tflat.dtype, pin_memory=True)
-        host_t.copy_(tflat, non_blocking=True)
-    copied = torch.cuda.Event()
-    copied.record()
-    result = launch()
-    copied.synchronize()
-    _check_offsets(host.numpy().astype(np.int64), documents.shape[0])
-    if host_t is not None:
-        _check_targets(host_t.numpy().astype(np.int64), nb)
-    return result
+        _check_targets(_to_host(targets)[0], flat.numel() - 1)
+    return launch()
 
 
 def score_contrastive(queries, documents, document_offsets) -> torch.Tensor:

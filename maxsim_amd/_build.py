@@ -27,7 +27,7 @@ ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 ARCH = os.environ.get("MAXSIM_AMD_ARCH", "gfx950")
 
 HIP_SOURCES = ["maxsim_fwd.hip", "maxsim_kloop.hip", "maxsim_bwd.hip", "maxsim_pack.hip",
-               "maxsim_ce.hip", "maxsim_capi.hip"]
+               "maxsim_ce.hip", "maxsim_check.hip", "maxsim_capi.hip"]
 LIB = PKG / "libmaxsim_amd.so"
 TORCH_LIB = PKG / "_maxsim_amd_torch.so"
 

@@ -27,6 +27,26 @@ int maxsim_internal_contrastive_forward(maxsim_dtype dtype, const void* queries,
                                         int32_t* argmax, void* workspace, size_t workspace_bytes,
                                         void* stream);
 
+/* One index array of a layout check: CSR offsets (strictly increasing from 0
+ * to `limit`), ids in [0, limit) or lengths in [1, limit]; int32 or int64. */
+enum maxsim_check_kind { MAXSIM_CHECK_CSR = 0, MAXSIM_CHECK_IDS = 1, MAXSIM_CHECK_LENGTHS = 2 };
+#define MAXSIM_CHECK_ARRAYS 4
+typedef struct {
+  const void* values; /* device memory */
+  int64_t n;
+  int64_t limit;
+  int kind;
+  int is64;
+} maxsim_check_array;
+
+/* Checks the arrays on `stream` and writes maxsim_internal_check_words() words
+ * of pinned host memory at `status`, which the caller has zeroed: bit 0 done,
+ * bit 1 a value is bad, bits 32 and up the longest segment of the first array
+ * if it holds CSR offsets. */
+int maxsim_internal_check_words(const maxsim_check_array* arrays, int count);
+int maxsim_internal_check_layout(const maxsim_check_array* arrays, int count, uint64_t* status,
+                                 void* stream);
+
 #ifdef __cplusplus
 }
 #endif

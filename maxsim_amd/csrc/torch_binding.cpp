@@ -12,6 +12,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
 
+#include <chrono>
 #include <optional>
 #include <tuple>
 #include <vector>
@@ -68,6 +69,101 @@ at::TensorOptions f32_opts(const Tensor& q) {
 }
 at::TensorOptions i32_opts(const Tensor& q) {
   return at::TensorOptions().dtype(at::kInt).device(q.device());
+}
+
+// ---- layout checks ---------------------------------------------------------
+
+// Queue the check of a call's index arrays on the current stream, ahead of
+// the call's kernels; the words of the result are for check_wait(), the last
+// one is the stream.  They are pinned memory that the kernel writes: every
+// begin is followed by a wait.  (On a stream of its own, behind an event, the
+// check gained nothing for the largest calls either, whose workgroups leave it
+// no room: 256 x 1000 candidates 1570 against 1565 us.)
+Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) {
+  std::vector<Tensor> held;
+  maxsim_check_array arrays[MAXSIM_CHECK_ARRAYS];
+  TORCH_CHECK(!checks.empty() && checks.size() <= MAXSIM_CHECK_ARRAYS, "layout check: arrays");
+  int n = 0;
+  for (const auto& [t, kind, limit] : checks) {
+    TORCH_CHECK(t.scalar_type() == at::kInt || t.scalar_type() == at::kLong,
+                "index tensors must be int32 or int64; got ", t.scalar_type());
+    held.push_back(t.contiguous());
+    const Tensor& c = held.back();
+    arrays[n++] = maxsim_check_array{c.numel() > 0 ? c.data_ptr() : nullptr, c.numel(), limit,
+                                     kind, c.scalar_type() == at::kLong ? 1 : 0};
+  }
+  const Tensor& first = held.front();
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(first.device());
+  const int words = maxsim_internal_check_words(arrays, n);
+  Tensor status =
+      at::empty({words + 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  int64_t* w = status.data_ptr<int64_t>();
+  for (int i = 0; i < words; ++i) w[i] = 0;
+  void* stream = current_stream(first);
+  w[words] = reinterpret_cast<intptr_t>(stream);
+  check_status(maxsim_internal_check_layout(arrays, n, reinterpret_cast<uint64_t*>(w), stream));
+  return status;
+}
+
+Tensor maxsim_check_padded(Tensor query_lengths, Tensor doc_lengths, int64_t Lq, int64_t Ld) {
+  return check_begin({{query_lengths, MAXSIM_CHECK_LENGTHS, Lq},
+                      {doc_lengths, MAXSIM_CHECK_LENGTHS, Ld}});
+}
+
+Tensor maxsim_check_packed(Tensor query_offsets, Tensor document_offsets, Tensor pair_query_ids,
+                           Tensor pair_document_ids, int64_t total_q, int64_t total_d) {
+  return check_begin({{query_offsets, MAXSIM_CHECK_CSR, total_q},
+                      {document_offsets, MAXSIM_CHECK_CSR, total_d},
+                      {pair_query_ids, MAXSIM_CHECK_IDS, query_offsets.numel() - 1},
+                      {pair_document_ids, MAXSIM_CHECK_IDS, document_offsets.numel() - 1}});
+}
+
+Tensor maxsim_check_contrastive(Tensor document_offsets, int64_t total_d,
+                                std::optional<Tensor> targets) {
+  if (targets.has_value())
+    return check_begin({{document_offsets, MAXSIM_CHECK_CSR, total_d},
+                        {*targets, MAXSIM_CHECK_IDS, document_offsets.numel() - 1}});
+  return check_begin({{document_offsets, MAXSIM_CHECK_CSR, total_d}});
+}
+
+// Wait for a check on `like`'s device: the longest
+// segment of its first array (0 unless CSR offsets), or -1 when a value is
+// bad.  Polls the words, and the stream every 100 ms (a query puts a marker
+// into it), so that an error there, or a stream that ended without the words,
+// ends the wait.
+int64_t maxsim_check_wait(Tensor status, Tensor like) {
+  const int64_t words = status.numel() - 1;
+  const int64_t* w = status.data_ptr<int64_t>();
+  const hipStream_t stream = reinterpret_cast<hipStream_t>(static_cast<intptr_t>(w[words]));
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
+  int64_t longest = 0;
+  bool bad = false;
+  constexpr std::chrono::milliseconds kLook{100};
+  auto look = std::chrono::steady_clock::now() + kLook;
+  for (int64_t i = 0; i < words; ++i) {
+    int64_t v = 0;
+    bool drained = false;
+    for (int64_t spins = 1;; ++spins) {
+      v = __atomic_load_n(w + i, __ATOMIC_ACQUIRE);
+      if (v & 1) break;
+      TORCH_CHECK(!drained, "maxsim_amd: the layout check did not report");
+      if (spins % 4096 == 0 && std::chrono::steady_clock::now() >= look) {
+        look = std::chrono::steady_clock::now() + kLook;
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();
+        } else {
+          TORCH_CHECK(e == hipSuccess, "maxsim_amd: HIP error: ", hipGetErrorString(e));
+          drained = true;  // one more look
+        }
+      } else {
+        __builtin_ia32_pause();
+      }
+    }
+    bad |= (v & 2) != 0;
+    longest = std::max(longest, (int64_t)((uint64_t)v >> 32));
+  }
+  return bad ? -1 : longest;
 }
 
 // ---- packed ---------------------------------------------------------------
@@ -634,6 +730,13 @@ TORCH_LIBRARY(maxsim_amd, m) {
   m.def("maxsim_packed_backward(Tensor dscore, Tensor queries, Tensor query_offsets, "
         "Tensor documents, Tensor document_offsets, Tensor pair_query_ids, "
         "Tensor pair_document_ids, Tensor argmax, int max_q_len) -> (Tensor, Tensor)");
+  // layout checks of the Python functions, not operators of the reference
+  m.def("maxsim_check_padded(Tensor query_lengths, Tensor doc_lengths, int Lq, int Ld) -> Tensor");
+  m.def("maxsim_check_packed(Tensor query_offsets, Tensor document_offsets, "
+        "Tensor pair_query_ids, Tensor pair_document_ids, int total_q, int total_d) -> Tensor");
+  m.def("maxsim_check_contrastive(Tensor document_offsets, int total_d, Tensor? targets) "
+        "-> Tensor");
+  m.def("maxsim_check_wait(Tensor status, Tensor like) -> int");
   m.def("maxsim_contrastive_forward(Tensor queries, Tensor documents, "
         "Tensor document_offsets) -> Tensor");
   m.def("maxsim_contrastive_forward_with_argmax(Tensor queries, Tensor documents, "
@@ -667,6 +770,10 @@ TORCH_LIBRARY_IMPL(maxsim_amd, CUDA, m) {
   m.impl("maxsim_packed_forward_with_argmax", &maxsim_packed_forward_with_argmax);
   m.impl("maxsim_packed_backward", &maxsim_packed_backward);
   m.impl("maxsim_packed_backward_typed", &maxsim_packed_backward_typed);
+  m.impl("maxsim_check_padded", &maxsim_check_padded);
+  m.impl("maxsim_check_packed", &maxsim_check_packed);
+  m.impl("maxsim_check_contrastive", &maxsim_check_contrastive);
+  m.impl("maxsim_check_wait", &maxsim_check_wait);
   m.impl("maxsim_contrastive_forward", &maxsim_contrastive_forward);
   m.impl("maxsim_contrastive_forward_with_argmax",
          &maxsim_contrastive_forward_with_argmax);

@@ -1,0 +1,107 @@
+"""The device-side layout check behind the Python functions: every array kind
+and index type, one to 64 workgroups, a bad value at either end, on workgroup
+boundaries and in each array, the longest segment, and the reference's errors."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import maxsim_amd
+from maxsim_amd._ops import ops
+
+from ._helpers import DEVICE, make_packed, make_padded
+
+pytestmark = pytest.mark.gpu
+
+
+def _found(status, like):
+    return ops.maxsim_check_wait(status, like)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("n", [1, 2, 1024, 8192, 8193, 70001, 700001])
+def test_check_lengths_and_ids(n, dtype):
+    gen = torch.Generator().manual_seed(n)
+    dlen = torch.randint(1, 51, (n,), generator=gen, dtype=dtype).to(DEVICE)
+    qlen = torch.tensor([7], dtype=dtype, device=DEVICE)
+    assert _found(ops.maxsim_check_padded(qlen, dlen, 7, 50), qlen) == 0
+    assert _found(ops.maxsim_check_padded(qlen, dlen, 6, 50), qlen) == -1
+    for at in {0, n // 2, n - 1}:
+        for value in (0, 51, -1, 2 ** 31 - 1):
+            bad = dlen.clone()
+            bad[at] = value
+            assert _found(ops.maxsim_check_padded(qlen, bad, 7, 50), qlen) == -1
+    if dtype == torch.int64:
+        bad = dlen.clone()
+        bad[n - 1] = 2 ** 32 + 1  # 1 if narrowed
+        assert _found(ops.maxsim_check_padded(qlen, bad, 7, 50), qlen) == -1
+    # not contiguous
+    wide = torch.zeros(n, 2, dtype=dtype, device=DEVICE)
+    wide[:, 0] = dlen
+    assert _found(ops.maxsim_check_padded(qlen, wide[:, 0], 7, 50), qlen) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("n", [1, 2, 1023, 8191, 8192, 100000])
+def test_check_offsets(n, dtype):
+    gen = torch.Generator().manual_seed(n)
+    lens = torch.randint(1, 9, (n,), generator=gen)
+    lens[n // 2] = 11
+    off = torch.zeros(n + 1, dtype=dtype)
+    off[1:] = lens.cumsum(0)
+    total = int(off[-1])
+    off = off.to(DEVICE)
+    assert _found(ops.maxsim_check_contrastive(off, total, None), off) == 11
+    assert _found(ops.maxsim_check_contrastive(off, total + 1, None), off) == -1
+    for at in {0, 1, n // 2, n}:
+        bad = off.clone()
+        bad[at] = total + 5 if at == 0 else off[at - 1]
+        assert _found(ops.maxsim_check_contrastive(bad, total, None), off) == -1
+    targets = torch.tensor([0, n - 1], device=DEVICE)
+    assert _found(ops.maxsim_check_contrastive(off, total, targets), off) == 11
+    assert _found(ops.maxsim_check_contrastive(off, total, targets + 1), off) == -1
+    one = off[:1].contiguous()
+    assert _found(ops.maxsim_check_contrastive(one, 0, None), off) == -1
+
+
+def test_check_packed_arrays_and_errors():
+    args = list(make_packed(6, 9, 40, 32, (1, 12), (1, 20), torch.float16, seed=1))
+    q, qo, d, do, qi, di = args
+    longest = int((qo[1:] - qo[:-1]).max())
+    status = ops.maxsim_check_packed(qo, do, qi, di, q.shape[0], d.shape[0])
+    assert _found(status, qo) == longest
+    scores, argmax = maxsim_amd.score_pairs_packed_with_argmax(*args)
+    assert tuple(argmax.shape) == (40, longest)
+    assert torch.equal(maxsim_amd.score_pairs_packed(*args), scores)
+    for which, value, word in [(1, -1, "query_offsets"), (3, -1, "document_offsets"),
+                               (4, 6, "pair_query_ids"), (5, 9, "pair_document_ids")]:
+        bad = [t.clone() for t in args]
+        bad[which][-1] = value
+        for kw in ({}, {"max_q_len": longest}):
+            with pytest.raises(RuntimeError, match=word):
+                maxsim_amd.score_pairs_packed_with_argmax(*bad, **kw)
+            with pytest.raises(RuntimeError, match=word):
+                maxsim_amd.score_pairs_packed(*bad, **kw)
+    with pytest.raises(ValueError, match="max_q_len"):
+        maxsim_amd.score_pairs_packed(*args, max_q_len=longest - 1)
+    torch.cuda.synchronize()
+
+
+def test_check_waits_when_the_launch_raises():
+    """A launch that fails leaves no check writing into a freed buffer: the
+    next calls, which reuse it, see their own verdicts."""
+    q, d, ql, dl = make_padded(2, 3, 4, 8, 16, torch.float32, seed=2)
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match="launch failed"):
+            status = ops.maxsim_check_padded(ql, dl, 4, 8)
+
+            def launch():
+                raise RuntimeError("launch failed")
+
+            maxsim_amd._run_checked(status, ql, launch)
+        bad = dl.clone()
+        bad[1, 2] = 9
+        with pytest.raises(ValueError, match="doc_lengths"):
+            maxsim_amd.score_candidates_padded(q, d, ql, bad)
+        maxsim_amd.score_candidates_padded(q, d, ql, dl)
