@@ -2172,6 +2172,18 @@ static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int
   if (r.tiled) return r;
   const int64_t nblk = (lq + kTileCols - 1) / kTileCols;
   if (!kloop_supported(dtype, dim, nblk)) return r;
+  // Few pairs: a workgroup (or wave) per pair, where the K-loop kernel's time
+  // is its longest document's, in one workgroup.  Documents of 47-428 rows,
+  // pair / K-loop kernels: bf16 dim 256, 256 pairs 11 / 27 us, 512 19 / 28,
+  // 960 31 / 28, with four blocks per query 32 pairs 35 / 26; fp32 dim 128,
+  // 992 pairs 52 / 72 us, 2025 73 / 87, 2400 of 300 queries 86 / 131, 3600 129
+  // / 104, with four blocks per query 256 pairs 55 / 72; fp32 dim 384, 32 pairs
+  // 123 / 199; bf16 dim 384, 32 pairs 48 / 36.
+  const int64_t cus = device_cus();
+  if (dtype == MAXSIM_FLOAT32
+          ? nblk <= 4 && nq * nb * nblk < 12 * cus
+          : dim <= kMaxRegDim && nblk <= 2 && nq * nb * nblk < 3 * cus)
+    return r;
   r.kloop = true;
   r.in_place = dim % kChunk == 0 && ptrs;
   r.copy_d = !(dim % kChunk == 0 && aligned16(d));

@@ -43,22 +43,24 @@ def _without_workspace(q, d, off):
     return s, a
 
 
+# enough pairs for the K-loop kernel: Nq * documents * blocks >= 768 (16-bit rows
+# up to 256), 3072 (fp32)
 @pytest.mark.parametrize("Nq,Lq,dim,d_lens,dtype", [
-    (9, 32, 80, [1, 32, 33, 128, 129, 40], BF16),        # one slice and one chunk
-    (9, 31, 96, [64] * 3 + [1] * 5, F16),
-    (3, 20, 256, [200, 97, 31], BF16),
+    (130, 32, 80, [1, 32, 33, 128, 129, 40], BF16),      # one slice and one chunk
+    (101, 31, 96, [64] * 3 + [1] * 5, F16),
+    (257, 20, 256, [200, 97, 31], BF16),
     (17, 32, 768, [5, 160], BF16),
-    (2, 33, 144, [300, 1, 129], F16),                     # blocks across waves
+    (129, 33, 144, [300, 1, 129], F16),                   # blocks across waves
     (3, 200, 160, [70, 33], BF16),                        # 7 of 8 blocks
     (1, 256, 160, [70, 33], BF16),                        # all 8
     (1, 257, 160, [70, 33], BF16),                        # one more than a workgroup holds
-    (5, 32, 128, [128, 1, 31, 96], F32),
-    (4, 40, 48, [33, 64, 2], F32),
-    (2, 8, 384, [50], F32),
+    (769, 32, 128, [128, 1, 31, 96], F32),
+    (513, 40, 48, [33, 64, 2], F32),
+    (5, 130, 384, [50, 9], F32),                          # five blocks
     (5, 32, 300, [33, 64, 2, 129], BF16),                 # rows that are copied
-    (3, 70, 100, [33, 64, 2], F16),
-    (3, 9, 101, [33, 64, 2], BF16),
-    (3, 9, 67, [33, 64, 2], F32),
+    (86, 70, 100, [33, 64, 2], F16),
+    (257, 9, 101, [33, 64, 2], BF16),
+    (1025, 9, 67, [33, 64, 2], F32),
 ])
 def test_kloop_forward(Nq, Lq, dim, d_lens, dtype):
     q, d, off = make_contrastive(Nq, Lq, dim, d_lens, dtype, seed=dim, unit=True)
@@ -90,7 +92,7 @@ def test_kloop_document_chunks(Nq, Lq, Nb, dim):
 
 @pytest.mark.parametrize("dim", [96, 100])
 def test_kloop_misaligned_rows_and_invalid_documents(dim):
-    q, d, off = make_contrastive(6, 32, dim, [20, 40, 10, 33, 50], BF16, seed=3, unit=True)
+    q, d, off = make_contrastive(160, 32, dim, [20, 40, 10, 33, 50], BF16, seed=3, unit=True)
     good, good_am = maxsim_amd.score_contrastive_with_argmax(q, d, off)
     shifted = torch.empty(d.numel() + 1, dtype=d.dtype, device=d.device)[1:].view_as(d)
     shifted.copy_(d)  # rows on a 2-byte boundary
@@ -106,7 +108,7 @@ def test_kloop_misaligned_rows_and_invalid_documents(dim):
 
 
 def test_kloop_nan_and_infinity():
-    q, d, off = make_contrastive(3, 32, 100, [40, 33, 70], BF16, seed=5, unit=True)
+    q, d, off = make_contrastive(260, 32, 100, [40, 33, 70], BF16, seed=5, unit=True)
     d[3, 7] = float("nan")
     d[45, 99] = float("inf")
     d[80, 0] = float("-inf")
