@@ -394,9 +394,12 @@ constexpr int kDqBatch = 4;
 constexpr int kDqSplitMaxDim = 2048;  // 8 * 256 slices: one row per workgroup at most
 constexpr int kDqTable = 2048;  // (row, document) pairs staged per chunk
 
-template <typename T, int U>
-__global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, bool vec, float* ws,
-                                                       int rows_per_group) {
+// VEC: 16-byte rows, a template parameter so that a batch's loads need no
+// branch between them (a join there waits for each): bf16, 300 x 300 documents
+// of 20-200 rows, whole backward at dim 768 460 -> 446 us, at dim 300 1985 ->
+// 450 us (rows on any boundary in whole fragments).
+template <typename T, int U, bool VEC>
+__global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, float* ws, int rows_per_group) {
   using S = typename T::storage;
   __shared__ int32_t t_src[kDqTable];  // [document in chunk][row in group]
   __shared__ float t_w[kDqTable];
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, bool vec, float
         for (int u = 0; u < U; ++u) {
           const int e = (MASKED ? min(bl + u, nc - 1) : bl + u) * rpg + local;
           wt[u] = t_w[e];
-          v[u] = load_frag<T>(D + (int64_t)t_src[e] * a.dim, k0, a.dim, vec);
+          v[u] = load_frag<T>(D + (int64_t)t_src[e] * a.dim, k0, a.dim, VEC);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -466,7 +469,7 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, bool vec, float
       if (bl < nc) batch(bl, std::true_type{});
     }
   }
-  if (active) store8f(ws + (int64_t)r * a.rows * a.dim + row * a.dim, k0, a.dim, vec, acc);
+  if (active) store8f(ws + (int64_t)r * a.rows * a.dim + row * a.dim, k0, a.dim, VEC, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -2508,8 +2511,9 @@ static void launch_dq_split(const DqArgs& a, bool vec, float* ws, bool vec_reduc
                             bool reduce, hipStream_t st) {
   const int rows_per_group = 256 / a.nslices;  // >= 8: dim <= 256
   const int64_t n_groups = (a.rows + rows_per_group - 1) / rows_per_group;
-  hipLaunchKernelGGL((dq_split_kernel<T, kDqBatch>), dim3((unsigned)(n_groups * kXcds)),
-                     dim3(256), 0, st, a, vec, ws, rows_per_group);
+  hipLaunchKernelGGL((vec ? dq_split_kernel<T, kDqBatch, true>
+                          : dq_split_kernel<T, kDqBatch, false>),
+                     dim3((unsigned)(n_groups * kXcds)), dim3(256), 0, st, a, ws, rows_per_group);
   if (!reduce) return;  // the dD launch adds the partial sums
   const int64_t n = a.rows * a.dim;
   const int64_t work = vec_reduce ? n / 4 : n;
@@ -2883,6 +2887,16 @@ static int contrastive_backward_impl(
   da.parts = 1;
   while (da.parts < 4 && q_bytes / da.parts > q_share && da.parts * 2 <= nslices)
     da.parts *= 2;
+  const int l2_parts = da.parts;
+  // Few documents: more parts, so that dd_contrastive_kernel's launch fills
+  // the chip; each buckets its document again, so of at least eight slices,
+  // or four below 128 workgroups.  Whole backward in bf16, with and without:
+  // 64 documents at dim 768 143 -> 66 us, 100 at dim 300 557 -> 125, 16 at dim
+  // 256 34 -> 14; 150 documents at dim 96 would go from 70 to 77 with parts of
+  // six slices.
+  while (da.parts < kXcds && num_documents * da.parts < 512 &&
+         nslices / (da.parts * 2) >= (num_documents * da.parts < 128 ? 4 : 8))
+    da.parts *= 2;
   da.part_slices = (nslices + da.parts - 1) / da.parts;
   da.group = 1;
   while (da.group < kDdMaxGroup && da.group < da.part_slices) da.group *= 2;
@@ -2931,7 +2945,7 @@ static int contrastive_backward_impl(
     // Few documents: more dimension parts (up to one per XCD), so that the
     // launch has about two workgroups per CU; each part buckets its
     // document's entries again, which costs little at such sizes.
-    int parts = da.parts;
+    int parts = l2_parts;
     while (parts < kXcds && num_documents * parts < 512 && nslices % (parts * 2) == 0)
       parts *= 2;
     const int g2 = nslices / parts;  // one slice per lane
