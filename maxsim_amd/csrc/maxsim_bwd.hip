@@ -498,16 +498,17 @@ constexpr int kWalkMaxRows = 32;   // rows per workgroup at most
 constexpr int kWalkPad = 4;        // table row stride = docs per stage + 4 (ints)
 constexpr int kWalkTableInts = kWalkTable + kWalkPad * kWalkMaxRows;
 
+// Row group `group` by 256 threads (tid) with the tables t_src and t_w of
+// kWalkTableInts each, 16-byte aligned; barriers, the same number for every
+// group, are the workgroup's.
 template <typename T, bool VEC, bool OFF32, typename O>
-__global__ __launch_bounds__(256) void dq_walk_kernel(DqArgs a, int rows_per_group) {
+__device__ __forceinline__ void dq_walk_rows(const DqArgs& a, int rows_per_group, int64_t group,
+                                             int tid, int32_t* t_src, float* t_w) {
   using S = typename T::storage;
-  __shared__ __align__(16) int32_t t_src[kWalkTableInts];
-  __shared__ __align__(16) float t_w[kWalkTableInts];
   const int R = rows_per_group;
   const int dps = kWalkTable / R;  // documents per stage, a multiple of 8
   const int stride = dps + kWalkPad;
-  const int tid = threadIdx.x;
-  const int64_t row0 = (int64_t)blockIdx.x * R;
+  const int64_t row0 = group * R;
   const int lr = tid / a.nslices;
   const int sl = tid - lr * a.nslices;
   const int64_t row = row0 + lr;
@@ -532,13 +533,17 @@ __global__ __launch_bounds__(256) void dq_walk_kernel(DqArgs a, int rows_per_gro
         f.hi = p[1];
       }
       return f;
-    } else if constexpr (OFF32) {
-      return load_frag<T>(reinterpret_cast<const S*>(Db + (uint32_t)src), k0, a.dim, VEC);
     } else {
-      return load_frag<T>(D + (int64_t)src * a.dim, k0, a.dim, VEC);
+      const S* r = OFF32 ? reinterpret_cast<const S*>(Db + (uint32_t)src)
+                         : D + (int64_t)src * a.dim;
+      if constexpr (VEC) return load_frag<T>(r, k0, a.dim, true);
+      // moved into place where it is added (place_frag)
+      return a.dim >= 8 ? load_frag_any<T>(r, k0, a.dim) : load_frag_short<T>(r, k0, a.dim);
     }
   };
-  auto add = [&](const Frag<T>& v, float w) {
+  const bool partial = !VEC && a.dim >= 8 && k0 + 8 > a.dim;
+  auto add = [&](Frag<T> v, float w) {
+    if (partial) place_frag<T>(v, k0, a.dim);
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = fmaf(w, frag_elem(v, e), acc[e]);
   };
@@ -599,6 +604,13 @@ __global__ __launch_bounds__(256) void dq_walk_kernel(DqArgs a, int rows_per_gro
     }
   }
   if (active) store8<O>(out_at<O>(a.dq, row * a.dim), k0, a.dim, VEC, acc);
+}
+
+template <typename T, bool VEC, bool OFF32, typename O>
+__global__ __launch_bounds__(256) void dq_walk_kernel(DqArgs a, int rows_per_group) {
+  __shared__ __align__(16) int32_t t_src[kWalkTableInts];
+  __shared__ __align__(16) float t_w[kWalkTableInts];
+  dq_walk_rows<T, VEC, OFF32, O>(a, rows_per_group, blockIdx.x, threadIdx.x, t_src, t_w);
 }
 
 // ---------------------------------------------------------------------------
@@ -885,8 +897,10 @@ __device__ __forceinline__ int div_small(int x, int d, float inv_d) {
 // entry pass (the host checks), since later passes add to the rows in fp32.
 // Rows before the first and after the last document are zeroed by part 0 of
 // the first and the last document.
+// `wg`: the workgroup's place in a grid of launch_dd's size (its residue mod
+// kXcds is its XCD's).
 template <typename T, bool VEC, int NS, typename O>
-__global__ __launch_bounds__(kDdThreads) void dd_contrastive_kernel(DdArgs a) {
+__device__ __forceinline__ void dd_contrastive_document(const DdArgs& a, unsigned wg) {
   using S = typename T::storage;
   extern __shared__ int lds_i[];
   const int R = a.rows_per_pass;
@@ -898,10 +912,10 @@ __global__ __launch_bounds__(kDdThreads) void dd_contrastive_kernel(DdArgs a) {
 
   // workgroup w -> XCD x = w % 8; part = x / (8 / parts); document
   // b = (w / 8) * (8 / parts) + x % (8 / parts)
-  const int xcd = blockIdx.x % kXcds;
+  const int xcd = wg % kXcds;
   const int per_part = kXcds / a.parts;
   const int part = xcd / per_part;
-  const int64_t b = (int64_t)(blockIdx.x / kXcds) * per_part + xcd % per_part;
+  const int64_t b = (int64_t)(wg / kXcds) * per_part + xcd % per_part;
   if (b >= a.nb) return;
   if (part == 0 && (b == 0 || b == a.nb - 1)) {
     const int64_t head = min(max((int64_t)a.doff[0], (int64_t)0), a.total_d);
@@ -1091,6 +1105,11 @@ __global__ __launch_bounds__(kDdThreads) void dd_contrastive_kernel(DdArgs a) {
   }
 }
 
+template <typename T, bool VEC, int NS, typename O>
+__global__ __launch_bounds__(kDdThreads) void dd_contrastive_kernel(DdArgs a) {
+  dd_contrastive_document<T, VEC, NS, O>(a, blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // dd, contrastive, the common case (dd_bucket_kernel): rows of 16-byte
 // fragments, dim <= 256 per part with an even number of 8-element slices,
@@ -1125,7 +1144,7 @@ constexpr int kBkClasses = 256;        // row size classes: ceil(entries / 4), c
 constexpr int kBkOrderMin = 4096;      // entries per document from which rows are ordered
 
 template <typename T, int NS, typename O>
-__device__ __forceinline__ void dd_bucket_document(DdArgs a) {
+__device__ __forceinline__ void dd_bucket_document(DdArgs a, unsigned wg) {
   using S = typename T::storage;
   extern __shared__ int lds_i[];
   const int R = a.rows_per_pass;
@@ -1137,11 +1156,11 @@ __device__ __forceinline__ void dd_bucket_document(DdArgs a) {
   int* cursor = start + (R + 1);      // [R + 1]
   int* ids = cursor + (R + 1);        // [E]
 
-  const int xcd = blockIdx.x % kXcds;
+  const int xcd = wg % kXcds;
   const int per_part = kXcds / a.parts;
   const int part = xcd / per_part;
   // place p of the grid (its workgroups: one per part)
-  const int64_t p = (int64_t)(blockIdx.x / kXcds) * per_part + xcd % per_part;
+  const int64_t p = (int64_t)(wg / kXcds) * per_part + xcd % per_part;
   if (p >= a.nb) return;
   if (part == 0 && (p == 0 || p == a.nb - 1)) {
     const int64_t head = min(max((int64_t)a.doff[0], (int64_t)0), a.total_d);
@@ -1468,8 +1487,50 @@ __global__ __launch_bounds__(kDdThreads) void dd_bucket_kernel(DdArgs a) {
   };
   constexpr bool kReduceFirst = O::bytes == 4;
   if (kReduceFirst && a.dq_ws) reduce_share();
-  dd_bucket_document<T, NS, O>(a);
+  dd_bucket_document<T, NS, O>(a, blockIdx.x);
   if (!kReduceFirst && a.dq_ws) reduce_share();
+}
+
+// ---------------------------------------------------------------------------
+// Both gradients of a small contrastive batch in one launch: dq_walk_rows and
+// the dd kernels do not depend on each other, and neither fills the chip for
+// long (64 queries x 64 documents: 12 and 15 us, one after the other).  The
+// first workgroups, whole XCD rows of them so that dd's keep their XCDs, take
+// two groups of query rows each, the others a document (and part).  LDS is
+// dynamic only: dd_bucket_document counts on starting at byte 0.
+// ---------------------------------------------------------------------------
+struct GradsArgs {
+  DqArgs dq;
+  DdArgs dd;
+  int walk_rows;     // rows per group
+  unsigned dq_wgs;   // multiple of kXcds
+};
+constexpr size_t kGradsWalkLds = 2 * 2 * kWalkTableInts * sizeof(int);
+
+template <typename T, bool VEC, typename O>
+__device__ __forceinline__ void grads_walk(const GradsArgs& g) {
+  extern __shared__ int lds_i[];
+  const int half = threadIdx.x >> 8;
+  int32_t* t_src = lds_i + half * 2 * kWalkTableInts;
+  dq_walk_rows<T, VEC, true, O>(g.dq, g.walk_rows, 2 * (int64_t)blockIdx.x + half,
+                                threadIdx.x & 255, t_src,
+                                reinterpret_cast<float*>(t_src + kWalkTableInts));
+}
+
+template <typename T, typename O>
+__global__ __launch_bounds__(kDdThreads) void grads_bucket_kernel(GradsArgs g) {
+  if (blockIdx.x < g.dq_wgs)
+    grads_walk<T, true, O>(g);
+  else
+    dd_bucket_document<T, 1, O>(g.dd, blockIdx.x - g.dq_wgs);
+}
+
+template <typename T, bool VEC, int NS, typename O>
+__global__ __launch_bounds__(kDdThreads) void grads_contrastive_kernel(GradsArgs g) {
+  if (blockIdx.x < g.dq_wgs)
+    grads_walk<T, VEC, O>(g);
+  else
+    dd_contrastive_document<T, VEC, NS, O>(g.dd, blockIdx.x - g.dq_wgs);
 }
 
 // ---------------------------------------------------------------------------
@@ -2444,6 +2505,16 @@ static int walk_rows(int nslices) {
   return r;
 }
 
+static GradsArgs grads_args(const DqArgs& dq, const DdArgs& dd) {
+  GradsArgs g{};
+  g.dq = dq;
+  g.dd = dd;
+  g.walk_rows = walk_rows(dq.nslices);
+  const int64_t per_wg = 2 * (int64_t)g.walk_rows;
+  g.dq_wgs = (unsigned)(((dq.rows + per_wg - 1) / per_wg + kXcds - 1) / kXcds * kXcds);
+  return g;
+}
+
 template <typename T>
 static void launch_dq_walk(const DqArgs& a, bool vec, bool off32, bool out16, hipStream_t st) {
   const int R = walk_rows(a.nslices);
@@ -2540,57 +2611,69 @@ static size_t max_lds_per_block() {
   return (size_t)cached[dev];
 }
 
-template <typename T, bool VEC, int NS, typename O>
-static int launch_dd_contrastive_v(const DdArgs& a, size_t lds, hipStream_t st) {
-  const auto kern = dd_contrastive_kernel<T, VEC, NS, O>;
-  if (lds > 64 * 1024) {
-    // once per device and instantiation: allow up to the device's maximum
-    static std::atomic<bool> raised[kMaxDevices];
-    if (int e = raise_lds_limit((const void*)kern, max_lds_per_block(), "dd_contrastive_kernel",
-                                raised))
-      return e;
-  }
-  const int64_t per_part = kXcds / a.parts;
-  const int64_t blocks = (a.nb + per_part - 1) / per_part * kXcds;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kDdThreads), lds, st, a);
+// dd alone, or (grads) with dq's row walk in the same launch.
+template <typename K, typename A>
+static int launch_grads(K kern, const A& args, int64_t blocks, size_t lds, const char* what,
+                        std::atomic<bool> (&raised)[kMaxDevices], hipStream_t st) {
+  if (lds > 64 * 1024)
+    if (int e = raise_lds_limit((const void*)kern, max_lds_per_block(), what, raised)) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kDdThreads), lds, st, args);
   return MAXSIM_OK;
 }
 
-template <typename T, typename O>
-static int launch_dd_bucket_o(const DdArgs& a, size_t lds, hipStream_t st) {
-  const auto kern = dd_bucket_kernel<T, 1, O>;
-  if (lds > 64 * 1024) {
-    static std::atomic<bool> raised[kMaxDevices];
-    if (int e = raise_lds_limit((const void*)kern, max_lds_per_block(), "dd_bucket_kernel",
-                                raised))
-      return e;
-  }
+template <typename T, bool VEC, int NS, typename O>
+static int launch_dd_contrastive_v(const DdArgs& a, const DqArgs* dq, size_t lds, hipStream_t st) {
   const int64_t per_part = kXcds / a.parts;
   const int64_t blocks = (a.nb + per_part - 1) / per_part * kXcds;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kDdThreads), lds, st, a);
-  return MAXSIM_OK;
+  if (dq) {
+    static std::atomic<bool> raised[kMaxDevices];
+    const GradsArgs g = grads_args(*dq, a);
+    return launch_grads(grads_contrastive_kernel<T, VEC, NS, O>, g, blocks + g.dq_wgs,
+                        std::max(lds, kGradsWalkLds), "grads_contrastive_kernel", raised, st);
+  }
+  // the limit is raised once per device and instantiation, to the device's maximum
+  static std::atomic<bool> raised[kMaxDevices];
+  return launch_grads(dd_contrastive_kernel<T, VEC, NS, O>, a, blocks, lds,
+                      "dd_contrastive_kernel", raised, st);
+}
+
+template <typename T, typename O>
+static int launch_dd_bucket_o(const DdArgs& a, const DqArgs* dq, size_t lds, hipStream_t st) {
+  const int64_t per_part = kXcds / a.parts;
+  const int64_t blocks = (a.nb + per_part - 1) / per_part * kXcds;
+  if (dq) {
+    static std::atomic<bool> raised[kMaxDevices];
+    const GradsArgs g = grads_args(*dq, a);
+    return launch_grads(grads_bucket_kernel<T, O>, g, blocks + g.dq_wgs,
+                        std::max(lds, kGradsWalkLds), "grads_bucket_kernel", raised, st);
+  }
+  static std::atomic<bool> raised[kMaxDevices];
+  return launch_grads(dd_bucket_kernel<T, 1, O>, a, blocks, lds, "dd_bucket_kernel", raised, st);
 }
 
 template <typename T>
-static int launch_dd_bucket(const DdArgs& a, size_t lds, bool out16, hipStream_t st) {
-  return out16 ? launch_dd_bucket_o<T, T>(a, lds, st) : launch_dd_bucket_o<T, F32>(a, lds, st);
+static int launch_dd_bucket(const DdArgs& a, const DqArgs* dq, size_t lds, bool out16,
+                            hipStream_t st) {
+  return out16 ? launch_dd_bucket_o<T, T>(a, dq, lds, st)
+               : launch_dd_bucket_o<T, F32>(a, dq, lds, st);
 }
 
 template <typename T, typename O>
-static int launch_dd_contrastive_o(const DdArgs& a, bool vec, size_t lds, hipStream_t st) {
+static int launch_dd_contrastive_o(const DdArgs& a, const DqArgs* dq, bool vec, size_t lds,
+                                   hipStream_t st) {
   const bool two = a.part_slices > a.group;
   if (vec)
-    return two ? launch_dd_contrastive_v<T, true, 2, O>(a, lds, st)
-               : launch_dd_contrastive_v<T, true, 1, O>(a, lds, st);
-  return two ? launch_dd_contrastive_v<T, false, 2, O>(a, lds, st)
-             : launch_dd_contrastive_v<T, false, 1, O>(a, lds, st);
+    return two ? launch_dd_contrastive_v<T, true, 2, O>(a, dq, lds, st)
+               : launch_dd_contrastive_v<T, true, 1, O>(a, dq, lds, st);
+  return two ? launch_dd_contrastive_v<T, false, 2, O>(a, dq, lds, st)
+             : launch_dd_contrastive_v<T, false, 1, O>(a, dq, lds, st);
 }
 
 template <typename T>
-static int launch_dd_contrastive(const DdArgs& a, bool vec, size_t lds, bool out16,
-                                 hipStream_t st) {
-  return out16 ? launch_dd_contrastive_o<T, T>(a, vec, lds, st)
-               : launch_dd_contrastive_o<T, F32>(a, vec, lds, st);
+static int launch_dd_contrastive(const DdArgs& a, const DqArgs* dq, bool vec, size_t lds,
+                                 bool out16, hipStream_t st) {
+  return out16 ? launch_dd_contrastive_o<T, T>(a, dq, vec, lds, st)
+               : launch_dd_contrastive_o<T, F32>(a, dq, vec, lds, st);
 }
 
 template <typename T>
@@ -3003,6 +3086,7 @@ static int contrastive_backward_impl(
   const size_t ws_need = maxsim_amd_contrastive_backward_workspace_size(num_queries, Lq, dim);
   // 32-bit byte offsets of D rows when D is below 2 GiB
   const bool off32 = total_d_tokens * dim * eb < ((int64_t)1 << 31);
+  const DqArgs* with_dd = nullptr;
   if (workspace && ws_need > 0 && workspace_bytes >= ws_need) {
     float* ws = static_cast<float*>(workspace);
     const bool vec_ws = vec && aligned16b(workspace);
@@ -3022,6 +3106,12 @@ static int contrastive_backward_impl(
       ba.dq_n = num_queries * Lq * dim;
       ba.dq_vec = vec_reduce ? 1 : 0;
     }
+  } else if (nslices <= 256 && off32 && grads_args(qa, da).dq_wgs <= (unsigned)device_cus()) {
+    // dq in the dd launch, while its workgroups leave most of the chip to
+    // dd's.  Whole backward, bf16, one launch / two: 64 x 64 documents at dim
+    // 128 (64 workgroups) 21 / 24.5 us, fp32 72 x 72 (72) 29 / 41; at dim 768
+    // (512) 76 / 65.
+    with_dd = &qa;
   } else if (nslices <= 256) {
     MAXSIM_DISPATCH(dtype, launch_dq_walk, qa, vec, off32, out16, st);
     if (int e = check_launch("dq_walk_kernel")) return e;
@@ -3031,15 +3121,17 @@ static int contrastive_backward_impl(
   }
 
   if (bucket) {
-    const int rc = dtype == MAXSIM_BFLOAT16 ? launch_dd_bucket<BF16>(ba, blds, out16, st)
-                   : dtype == MAXSIM_FLOAT16 ? launch_dd_bucket<F16>(ba, blds, out16, st)
-                                             : launch_dd_bucket<F32>(ba, blds, out16, st);
+    const int rc =
+        dtype == MAXSIM_BFLOAT16 ? launch_dd_bucket<BF16>(ba, with_dd, blds, out16, st)
+        : dtype == MAXSIM_FLOAT16 ? launch_dd_bucket<F16>(ba, with_dd, blds, out16, st)
+                                  : launch_dd_bucket<F32>(ba, with_dd, blds, out16, st);
     if (rc) return rc;
     return check_launch("dd_bucket_kernel");
   }
-  const int rc = dtype == MAXSIM_BFLOAT16 ? launch_dd_contrastive<BF16>(da, vec, lds, out16, st)
-                 : dtype == MAXSIM_FLOAT16 ? launch_dd_contrastive<F16>(da, vec, lds, out16, st)
-                                           : launch_dd_contrastive<F32>(da, vec, lds, out16, st);
+  const int rc =
+      dtype == MAXSIM_BFLOAT16 ? launch_dd_contrastive<BF16>(da, with_dd, vec, lds, out16, st)
+      : dtype == MAXSIM_FLOAT16 ? launch_dd_contrastive<F16>(da, with_dd, vec, lds, out16, st)
+                                : launch_dd_contrastive<F32>(da, with_dd, vec, lds, out16, st);
   if (rc) return rc;
   return check_launch("dd_contrastive_kernel");
 }
