@@ -11,7 +11,7 @@ import maxsim_amd
 from maxsim_amd._ops import ops
 from oracle import maxsim_oracle as oracle
 
-from ._helpers import (DTYPES, SCORE_TOL, assert_close, check_argmax, make_packed, make_padded,
+from ._helpers import (DTYPES, GRAD_TOL, SCORE_TOL, assert_close, check_argmax, make_packed, make_padded,
                        np64, npi)
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +54,25 @@ def test_packed_forward_row_widths_many_pairs(dim, dtype):
     s_ref, _ = oracle.packed_forward(np64(q), npi(qo), np64(d), npi(do), npi(qi), npi(di), 40)
     tol = dict(SCORE_TOL[dtype], atol=SCORE_TOL[dtype]["atol"] * max(1.0, dim / 64))
     assert_close(s, s_ref, **tol)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("B,C,Lq,Ld,dim", [
+    (3, 5, 20, 40, 100), (2, 40, 9, 17, 128), (1, 300, 5, 12, 67), (4, 3, 70, 33, 300),
+    (2, 16, 1, 1, 8), (2, 17, 33, 40, 5),
+])
+def test_padded_backward_row_widths(B, C, Lq, Ld, dim, dtype):
+    """Both padded gradients of one launch, fp32 and in the inputs' dtype, with
+    one to eight lanes per query row and candidates that are not a multiple of
+    the gathers in flight; padding rows are zero."""
+    q, d, ql, dl = make_padded(B, C, Lq, Ld, dim, dtype, seed=dim + C)
+    _, a = maxsim_amd.score_candidates_padded_with_argmax(q, d, ql, dl)
+    g = torch.randn(B, C, generator=torch.Generator().manual_seed(C))
+    flat = (g.to(q.device).reshape(-1), q.reshape(B * Lq, dim), d.reshape(B * C * Ld, dim), ql,
+            dl.reshape(-1), a, Lq, Ld, C)
+    dq, dd = ops.maxsim_padded_backward(*flat)
+    dq_ref, dd_ref = oracle.padded_backward(np64(g), np64(q), np64(d), npi(ql), npi(dl), npi(a))
+    assert_close(dq.view(q.shape), dq_ref, **GRAD_TOL[dtype])
+    assert_close(dd.view(d.shape), dd_ref, **GRAD_TOL[dtype])
+    dq16, dd16 = ops.maxsim_padded_backward_typed(*flat)
+    assert torch.equal(dq16, dq.to(dtype)) and torch.equal(dd16, dd.to(dtype))
