@@ -2063,17 +2063,16 @@ __global__ __launch_bounds__(256) void packed_init_kernel(int32_t* groups, int64
   outside(dd, doff, nd, total_d);
 }
 
-// dq: workgroup = (query qi, block of its tokens); thread = (token row,
-// 8-element slice).
+// dq: workgroup = (query qi, block `tok_block` of its tokens); thread = (token
+// row, 8-element slice).
 template <typename T, bool VEC, typename O>
-__global__ __launch_bounds__(kGroupThreads) void dq_packed_kernel(PackedBwdArgs a,
-                                                                  PackedGroups g) {
+__device__ __forceinline__ void dq_packed_rows(const PackedBwdArgs& a, const PackedGroups& g,
+                                               int64_t qi, int tok_block) {
   using S = typename T::storage;
   __shared__ int64_t st_ds[kPairStage];
   __shared__ int32_t st_ld[kPairStage];
   __shared__ int32_t st_p[kPairStage];
   __shared__ float st_g[kPairStage];
-  const int64_t qi = blockIdx.x;
   const int64_t qs = a.qoff[qi], qe = a.qoff[qi + 1];
   if (qs < 0 || qe <= qs || qe > a.total_q) return;
   const int lq = (int)(qe - qs);
@@ -2082,8 +2081,8 @@ __global__ __launch_bounds__(kGroupThreads) void dq_packed_kernel(PackedBwdArgs 
   // rounds of kGroupThreads slices, one row per workgroup
   const int ns = min(a.nslices, kGroupThreads);
   const int rows_per_pass = kGroupThreads / ns;
-  // token block of this workgroup (grid.y covers max_q_len)
-  const int i0 = blockIdx.y * rows_per_pass;
+  // token block of this workgroup (the blocks cover max_q_len)
+  const int i0 = tok_block * rows_per_pass;
   if (i0 >= lq) return;
   const int local = tid / ns;
   const int k_lo = g.qstart[qi], k_hi = g.qstart[qi + 1];
@@ -2152,7 +2151,7 @@ constexpr int kPkRows = 1024;     // rows bucketed per pass
 constexpr int kPkEntries = 2048;  // entries per stage (bucket ids held in LDS)
 
 // True when a document with n_pairs pairs needs more than one stage of
-// entries in dd_packed_kernel.
+// entries in dd_packed_document.
 __device__ __forceinline__ bool dd_packed_multi_stage(const PackedBwdArgs& a, int n_pairs) {
   const int tc = min(a.slots, kPkEntries);
   return a.slots > tc || n_pairs > min(kPairStage, kPkEntries / tc);
@@ -2165,12 +2164,14 @@ __device__ __forceinline__ bool dd_packed_multi_stage(const PackedBwdArgs& a, in
 // us.  fp32 rows are bound by their writes, and the same bound cost 10 us
 // there (294.5 -> 304.6 us), so they keep the compiler's allocation, as do
 // unaligned rows (element loads: 148 VGPRs, whose cap would spill 47).
+// (Four waves for fp32 rows: with dq in the same kernel the compiler would
+// take 139 registers for fp32 inputs, three waves.)
 template <bool VEC, int NS, typename O>
-constexpr int kPkMinWaves = (VEC && NS == 1 && O::bytes == 2) ? 5 : 1;
+constexpr int kPkMinWaves = (VEC && NS == 1) ? (O::bytes == 2 ? 5 : 4) : 1;
 
 template <typename T, bool VEC, int NS, typename O>
-__global__ __launch_bounds__(kGroupThreads, (kPkMinWaves<VEC, NS, O>)) void dd_packed_kernel(
-    PackedBwdArgs a, PackedGroups g, int G) {
+__device__ __forceinline__ void dd_packed_document(const PackedBwdArgs& a, const PackedGroups& g,
+                                                   int G, int64_t di) {
   using S = typename T::storage;
   __shared__ int start[kPkRows + 1];
   __shared__ int cursor[kPkRows + 1];
@@ -2180,7 +2181,6 @@ __global__ __launch_bounds__(kGroupThreads, (kPkMinWaves<VEC, NS, O>)) void dd_p
   __shared__ int32_t st_p[kPairStage];
   __shared__ float st_g[kPairStage];
   __shared__ int n_full;  // rows with entries in this stage
-  const int64_t di = blockIdx.x;
   const int64_t ds = a.doff[di], de = a.doff[di + 1];
   if (ds < 0 || de <= ds || de > a.total_d) return;
   const int ld = (int)(de - ds);
@@ -2383,7 +2383,35 @@ __global__ __launch_bounds__(kGroupThreads, (kPkMinWaves<VEC, NS, O>)) void dd_p
   }
 }
 
-// dd with a 16-bit output type O for the documents dd_packed_kernel leaves
+// dq alone, on a (queries, token blocks) grid.
+template <typename T, bool VEC, typename O>
+__global__ __launch_bounds__(kGroupThreads) void dq_packed_kernel(PackedBwdArgs a,
+                                                                  PackedGroups g) {
+  dq_packed_rows<T, VEC, O>(a, g, blockIdx.x, blockIdx.y);
+}
+
+// Both packed gradients in one launch, the first n_dq workgroups (queries x
+// token blocks) for dq: dq waits on gathers, dd on a chain of dependent loads
+// and its writes.  Whole backward, two launches / one: 20,000 pairs of 512
+// queries and 8192 documents bf16 168 / 160 us, bf16 with fp32 gradients 301 /
+// 287, fp32 298 / 295; 777 pairs at dim 96 43 / 35; 4000 pairs at dim 300 281 /
+// 219.  dq's workgroups spread evenly among dd's instead: 164, 246, 365, 35, 225.
+// Rows of two slices per lane keep two launches (n_dq = 0 here): at dd's
+// registers dq has too few waves (fp32 dim 384 335 / 375).
+template <typename T, bool VEC, int NS, typename O>
+__global__ __launch_bounds__(kGroupThreads, (kPkMinWaves<VEC, NS, O>)) void grads_packed_kernel(
+    PackedBwdArgs a, PackedGroups g, int G, int64_t n_dq) {
+  const int64_t b = blockIdx.x;
+  if constexpr (NS == 1) {
+    if (b < n_dq) {
+      dq_packed_rows<T, VEC, O>(a, g, b % a.nq, (int)(b / a.nq));
+      return;
+    }
+  }
+  dd_packed_document<T, VEC, NS, O>(a, g, G, b - n_dq);
+}
+
+// dd with a 16-bit output type O for the documents dd_packed_document leaves
 // (those needing more than one stage of entries).  Workgroups stride over
 // blocks of 256 documents, list the block's documents that need this kernel
 // (one thread per document), and process the listed ones.  Rows are taken
@@ -2733,29 +2761,22 @@ static void launch_padded(const DqArgs& q, const PaddedDdArgs& a, bool vec, bool
 template <typename T, typename O>
 static void launch_packed_grouped_o(const PackedBwdArgs& a, const PackedGroups& g, bool vec,
                                     int G, hipStream_t st) {
-  if (a.nq > 0) {
-    const int rows_per_pass = kGroupThreads / std::min(a.nslices, kGroupThreads);
-    const dim3 grid((unsigned)a.nq, (unsigned)((a.slots + rows_per_pass - 1) / rows_per_pass));
-    if (vec)
-      hipLaunchKernelGGL((dq_packed_kernel<T, true, O>), grid, dim3(kGroupThreads), 0, st, a, g);
-    else
-      hipLaunchKernelGGL((dq_packed_kernel<T, false, O>), grid, dim3(kGroupThreads), 0, st, a, g);
-  }
+  const bool two = a.nslices > G;
+  const auto kern = vec ? (two ? grads_packed_kernel<T, true, 2, O> : grads_packed_kernel<T, true, 1, O>)
+                        : (two ? grads_packed_kernel<T, false, 2, O>
+                               : grads_packed_kernel<T, false, 1, O>);
+  const int rows_per_pass = kGroupThreads / std::min(a.nslices, kGroupThreads);
+  const int64_t blocks = (a.slots + rows_per_pass - 1) / rows_per_pass;
+  const int64_t n_dq = a.nq * blocks;
+  const bool one = !two && n_dq + a.nd <= kMaxBlocks256;
+  if (!one && a.nq > 0)
+    hipLaunchKernelGGL((vec ? dq_packed_kernel<T, true, O> : dq_packed_kernel<T, false, O>),
+                       dim3((unsigned)a.nq, (unsigned)blocks), dim3(kGroupThreads), 0, st, a, g);
+  const int64_t wgs = (one ? n_dq : 0) + a.nd;
+  if (wgs > 0)
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(kGroupThreads), 0, st, a, g, G,
+                       one ? n_dq : (int64_t)0);
   if (a.nd > 0) {
-    const bool two = a.nslices > G;
-    const dim3 grid((unsigned)a.nd);
-    if (vec && two)
-      hipLaunchKernelGGL((dd_packed_kernel<T, true, 2, O>), grid, dim3(kGroupThreads), 0, st, a,
-                         g, G);
-    else if (vec)
-      hipLaunchKernelGGL((dd_packed_kernel<T, true, 1, O>), grid, dim3(kGroupThreads), 0, st, a,
-                         g, G);
-    else if (two)
-      hipLaunchKernelGGL((dd_packed_kernel<T, false, 2, O>), grid, dim3(kGroupThreads), 0, st, a,
-                         g, G);
-    else
-      hipLaunchKernelGGL((dd_packed_kernel<T, false, 1, O>), grid, dim3(kGroupThreads), 0, st, a,
-                         g, G);
     if constexpr (O::bytes != 4) {
       const dim3 grid_m((unsigned)std::min<int64_t>((a.nd + kGroupThreads - 1) / kGroupThreads,
                                                     1024));
@@ -2942,7 +2963,7 @@ static int packed_backward_impl(
   const int G = pow2_at_least(nslices < 16 ? nslices : 16);  // lanes per dd row
   const bool vec_g = vec && aligned16b(dqueries) && aligned16b(ddocuments);
   MAXSIM_DISPATCH(dtype, launch_packed_grouped, a, g, vec_g, G, out16, st);
-  return check_launch("dq_packed_kernel / dd_packed_kernel");
+  return check_launch("grads_packed_kernel");
 }
 
 static int contrastive_backward_impl(
