@@ -21,55 +21,80 @@ namespace maxsim {
 // stream and numpy checks.
 // ---------------------------------------------------------------------------
 constexpr int kCheckThreads = 256;
-constexpr int kCheckPerThread = 8;   // values per thread from which another workgroup is taken
+constexpr int kCheckUnroll = 4;      // values in flight per thread
 constexpr int kCheckMaxWgs = 128;
 
 struct CheckArray {
   const void* p;
   int64_t n;
   int64_t limit;   // CSR: the last value; ids: below it; lengths: at most it
+  int first_wg;    // its workgroups: first_wg .. the next array's
   int kind;        // maxsim_check_kind
   bool is64;
 };
 struct CheckArgs {
   CheckArray a[MAXSIM_CHECK_ARRAYS];
   int count;
+  int64_t per_wg;  // values per workgroup, a multiple of kCheckThreads * kCheckUnroll
   uint64_t* status;
 };
+
+// A workgroup checks a run of one array, kCheckUnroll loads in flight per
+// thread (clamped, so that no branch keeps one waiting for another): 57,000
+// values of four arrays 8.8 us when every thread went through all of them.
+template <typename I>
+__device__ __forceinline__ bool check_run(const CheckArray& a, int64_t lo, int64_t hi,
+                                          int64_t& longest) {
+  const I* v = static_cast<const I*>(a.p);
+  bool bad = false;
+  if (a.kind == MAXSIM_CHECK_CSR) {
+    // pair i: values i and i + 1
+    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kCheckThreads * kCheckUnroll) {
+      int64_t x[kCheckUnroll], y[kCheckUnroll];
+#pragma unroll
+      for (int u = 0; u < kCheckUnroll; ++u) {
+        const int64_t i = min(i0 + u * kCheckThreads, hi - 1);
+        x[u] = v[i];
+        y[u] = v[i + 1];
+      }
+#pragma unroll
+      for (int u = 0; u < kCheckUnroll; ++u) {
+        const int64_t i = min(i0 + u * kCheckThreads, hi - 1);
+        bad |= y[u] <= x[u] || (i == 0 && x[u] != 0) || (i + 2 == a.n && y[u] != a.limit);
+        longest = max(longest, y[u] - x[u]);
+      }
+    }
+  } else {
+    const int64_t least = a.kind == MAXSIM_CHECK_IDS ? 0 : 1;
+    const int64_t most = a.kind == MAXSIM_CHECK_IDS ? a.limit - 1 : a.limit;
+    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kCheckThreads * kCheckUnroll) {
+      int64_t x[kCheckUnroll];
+#pragma unroll
+      for (int u = 0; u < kCheckUnroll; ++u) x[u] = v[min(i0 + u * kCheckThreads, hi - 1)];
+#pragma unroll
+      for (int u = 0; u < kCheckUnroll; ++u) bad |= x[u] < least || x[u] > most;
+    }
+  }
+  return bad;
+}
 
 __global__ __launch_bounds__(kCheckThreads) void check_layout_kernel(CheckArgs c) {
   __shared__ int any_bad, longest;
   if (threadIdx.x == 0) any_bad = longest = 0;
   __syncthreads();
-  bool bad = false;
+  int k = 0;
+  while (k + 1 < c.count && (int)blockIdx.x >= c.a[k + 1].first_wg) ++k;
+  const CheckArray a = c.a[k];
+  // entries: pairs of neighbours for CSR offsets, values otherwise
+  const int64_t n = a.kind == MAXSIM_CHECK_CSR ? a.n - 1 : a.n;
+  const int64_t lo = (int64_t)((int)blockIdx.x - a.first_wg) * c.per_wg;
+  const int64_t hi = min(lo + c.per_wg, n);
   int64_t seg = 0;
-  const int64_t first = (int64_t)blockIdx.x * kCheckThreads + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * kCheckThreads;
-  for (int k = 0; k < c.count; ++k) {
-    const CheckArray a = c.a[k];
-    auto at = [&](int64_t i) __attribute__((always_inline)) -> int64_t {
-      return a.is64 ? static_cast<const int64_t*>(a.p)[i] : static_cast<const int32_t*>(a.p)[i];
-    };
-    if (a.kind == MAXSIM_CHECK_CSR) {
-      if (a.n < 2) bad = true;
-#pragma unroll 4
-      for (int64_t i = first; i + 1 < a.n; i += stride) {
-        const int64_t lo = at(i), hi = at(i + 1);
-        bad |= hi <= lo || (i == 0 && lo != 0) || (i + 2 == a.n && hi != a.limit);
-        if (k == 0) seg = max(seg, hi - lo);
-      }
-    } else {
-      const int64_t least = a.kind == MAXSIM_CHECK_IDS ? 0 : 1;
-      const int64_t most = a.kind == MAXSIM_CHECK_IDS ? a.limit - 1 : a.limit;
-#pragma unroll 4
-      for (int64_t i = first; i < a.n; i += stride) {
-        const int64_t v = at(i);
-        bad |= v < least || v > most;
-      }
-    }
-  }
+  bool bad = a.kind == MAXSIM_CHECK_CSR && a.n < 2;
+  if (lo < hi)
+    bad |= a.is64 ? check_run<int64_t>(a, lo, hi, seg) : check_run<int32_t>(a, lo, hi, seg);
   // segments beyond 2^31 - 1 belong to arrays that are bad anyway
-  const int s = (int)(seg < 0x7fffffff ? seg : 0x7fffffff);
+  const int s = k == 0 ? (int)(seg < 0x7fffffff ? seg : 0x7fffffff) : 0;
   if (bad) any_bad = 1;
   if (s > 0) atomicMax(&longest, s);
   __syncthreads();
@@ -79,6 +104,22 @@ __global__ __launch_bounds__(kCheckThreads) void check_layout_kernel(CheckArgs c
                        __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Workgroups of each array (at least one) at `per_wg` values each.
+static int array_wgs(int64_t n, int64_t per_wg) {
+  return (int)std::max<int64_t>((n + per_wg - 1) / per_wg, 1);
+}
+static int64_t values_per_wg(const maxsim_check_array* arrays, int count, int* wgs) {
+  for (int64_t per = kCheckThreads * kCheckUnroll;; per *= 2) {
+    int64_t all = 0;
+    for (int k = 0; k < count; ++k) all += (arrays[k].n + per - 1) / per + 1;
+    if (all <= kCheckMaxWgs) {
+      *wgs = 0;
+      for (int k = 0; k < count; ++k) *wgs += array_wgs(arrays[k].n, per);
+      return per;
+    }
+  }
+}
+
 }  // namespace maxsim
 
 using namespace maxsim;
@@ -86,10 +127,9 @@ using namespace maxsim;
 extern "C" {
 
 int maxsim_internal_check_words(const maxsim_check_array* arrays, int count) {
-  int64_t n = 0;
-  for (int k = 0; k < count; ++k) n += arrays[k].n;
-  const int64_t per = (int64_t)kCheckThreads * kCheckPerThread;
-  return (int)std::min<int64_t>(std::max<int64_t>((n + per - 1) / per, 1), kCheckMaxWgs);
+  int wgs = 0;
+  values_per_wg(arrays, count, &wgs);
+  return wgs;
 }
 
 int maxsim_internal_check_layout(const maxsim_check_array* arrays, int count, uint64_t* status,
@@ -98,15 +138,18 @@ int maxsim_internal_check_layout(const maxsim_check_array* arrays, int count, ui
   if (count < 1 || count > MAXSIM_CHECK_ARRAYS || !status)
     return fail(MAXSIM_ERR_INVALID, "layout check: bad arguments");
   CheckArgs c{};
+  int wgs = 0;
+  c.per_wg = values_per_wg(arrays, count, &wgs);
+  int first = 0;
   for (int k = 0; k < count; ++k) {
     if (arrays[k].n > 0 && !arrays[k].values)
       return fail(MAXSIM_ERR_INVALID, "layout check: null array");
-    c.a[k] = CheckArray{arrays[k].values, arrays[k].n, arrays[k].limit, arrays[k].kind,
+    c.a[k] = CheckArray{arrays[k].values, arrays[k].n, arrays[k].limit, first, arrays[k].kind,
                         arrays[k].is64 != 0};
+    first += array_wgs(arrays[k].n, c.per_wg);
   }
   c.count = count;
   c.status = status;
-  const int wgs = maxsim_internal_check_words(arrays, count);
   hipLaunchKernelGGL(check_layout_kernel, dim3((unsigned)wgs), dim3(kCheckThreads), 0,
                      static_cast<hipStream_t>(stream), c);
   return check_launch("check_layout_kernel");
