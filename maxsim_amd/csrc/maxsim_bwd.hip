@@ -2391,13 +2391,16 @@ __global__ __launch_bounds__(kGroupThreads) void dq_packed_kernel(PackedBwdArgs 
 }
 
 // Both packed gradients in one launch, the first n_dq workgroups (queries x
-// token blocks) for dq: dq waits on gathers, dd on a chain of dependent loads
-// and its writes.  Whole backward, two launches / one: 20,000 pairs of 512
-// queries and 8192 documents bf16 168 / 160 us, bf16 with fp32 gradients 301 /
-// 287, fp32 298 / 295; 777 pairs at dim 96 43 / 35; 4000 pairs at dim 300 281 /
-// 219.  dq's workgroups spread evenly among dd's instead: 164, 246, 365, 35, 225.
-// Rows of two slices per lane keep two launches (n_dq = 0 here): at dd's
-// registers dq has too few waves (fp32 dim 384 335 / 375).
+// token blocks) for dq, where those are few (at most four per CU): dq waits on
+// gathers, dd on a chain of dependent loads and its writes.  Whole backward,
+// two launches / one: bf16 777 pairs at dim 96 (244 workgroups) 43 / 35 us,
+// 4000 pairs at dim 300 281 / 219, fp32 9000 pairs (900) 91 / 79.  With 2048 of
+// them (20,000 pairs of 512 queries and 8192 documents) dq fills the chip
+// first, at dd's five waves per SIMD instead of eight: 168 / 160 us on the same
+// inputs again and again, but 154 / 162 us for the two kernels in a training
+// step, whose rows come from HBM.  Rows of two slices per lane keep two
+// launches (n_dq = 0 here): at dd's registers dq has too few waves (fp32 dim
+// 384 335 / 375).
 template <typename T, bool VEC, int NS, typename O>
 __global__ __launch_bounds__(kGroupThreads, (kPkMinWaves<VEC, NS, O>)) void grads_packed_kernel(
     PackedBwdArgs a, PackedGroups g, int G, int64_t n_dq) {
@@ -2768,7 +2771,7 @@ static void launch_packed_grouped_o(const PackedBwdArgs& a, const PackedGroups& 
   const int rows_per_pass = kGroupThreads / std::min(a.nslices, kGroupThreads);
   const int64_t blocks = (a.slots + rows_per_pass - 1) / rows_per_pass;
   const int64_t n_dq = a.nq * blocks;
-  const bool one = !two && n_dq + a.nd <= kMaxBlocks256;
+  const bool one = !two && n_dq <= 4 * (int64_t)device_cus() && n_dq + a.nd <= kMaxBlocks256;
   if (!one && a.nq > 0)
     hipLaunchKernelGGL((vec ? dq_packed_kernel<T, true, O> : dq_packed_kernel<T, false, O>),
                        dim3((unsigned)a.nq, (unsigned)blocks), dim3(kGroupThreads), 0, st, a, g);
