@@ -11,7 +11,10 @@ gradients in a separate pass.  ``maxsim_pack_padded_rows`` is the device
 copy behind :func:`maxsim_amd._pack_padded` (padded -> packed rows), and
 ``maxsim_cross_entropy_forward`` / ``maxsim_contrastive_cross_entropy_backward``
 are the fused training loss behind
-:func:`maxsim_amd.score_contrastive_cross_entropy`.
+:func:`maxsim_amd.score_contrastive_cross_entropy`.  ``maxsim_check_padded``,
+``maxsim_check_packed`` and ``maxsim_check_contrastive`` queue a device-side
+check of a call's offsets, ids or lengths and return the words that
+``maxsim_check_wait`` waits for.
 
 Importing this module loads ``_maxsim_amd_torch.so`` (which pulls in
 ``libmaxsim_amd.so``).  There is no fallback: if the native build is missing
