@@ -73,18 +73,29 @@ at::TensorOptions i32_opts(const Tensor& q) {
 
 // ---- layout checks ---------------------------------------------------------
 
+// Marks the words at `w` as a check's: a tensor from elsewhere, or a copy,
+// would be waited for in vain and its last words taken for a stream.
+int64_t check_tag(const int64_t* w, int64_t words) {
+  return (int64_t)(reinterpret_cast<uintptr_t>(w) ^ (0x6d617873696d0000ull + (uint64_t)words));
+}
+
 // Queue the check of a call's index arrays on the current stream, ahead of
 // the call's kernels; the words of the result are for check_wait(), the last
-// one is the stream.  They are pinned memory that the kernel writes: every
-// begin is followed by a wait.  (On a stream of its own, behind an event, the
-// check gained nothing for the largest calls either, whose workgroups leave it
-// no room: 256 x 1000 candidates 1570 against 1565 us.)
+// two are the stream and a tag that only these results have.  They are pinned
+// memory that the kernel writes: every begin is followed by a wait.  (On a
+// stream of its own, behind an event, the check gained nothing for the largest
+// calls either, whose workgroups leave it no room: 256 x 1000 candidates 1570
+// against 1565 us.)
 Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) {
   std::vector<Tensor> held;
   maxsim_check_array arrays[MAXSIM_CHECK_ARRAYS];
   TORCH_CHECK(!checks.empty() && checks.size() <= MAXSIM_CHECK_ARRAYS, "layout check: arrays");
   int n = 0;
+  const at::Device device = std::get<0>(checks.front()).device();
   for (const auto& [t, kind, limit] : checks) {
+    TORCH_CHECK(t.device().is_cuda() && t.device() == device,
+                "index tensors must be on one HIP (torch 'cuda') device; got ", device, " and ",
+                t.device());
     TORCH_CHECK(t.scalar_type() == at::kInt || t.scalar_type() == at::kLong,
                 "index tensors must be int32 or int64; got ", t.scalar_type());
     held.push_back(t.contiguous());
@@ -96,11 +107,12 @@ Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) 
   c10::hip::HIPGuardMasqueradingAsCUDA guard(first.device());
   const int words = maxsim_internal_check_words(arrays, n);
   Tensor status =
-      at::empty({words + 1}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+      at::empty({words + 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   int64_t* w = status.data_ptr<int64_t>();
   for (int i = 0; i < words; ++i) w[i] = 0;
   void* stream = current_stream(first);
   w[words] = reinterpret_cast<intptr_t>(stream);
+  w[words + 1] = check_tag(w, words);
   check_status(maxsim_internal_check_layout(arrays, n, reinterpret_cast<uint64_t*>(w), stream));
   return status;
 }
@@ -126,14 +138,19 @@ Tensor maxsim_check_contrastive(Tensor document_offsets, int64_t total_d,
   return check_begin({{document_offsets, MAXSIM_CHECK_CSR, total_d}});
 }
 
-// Wait for a check on `like`'s device: the longest
-// segment of its first array (0 unless CSR offsets), or -1 when a value is
-// bad.  Polls the words, and the stream every 100 ms (a query puts a marker
-// into it), so that an error there, or a stream that ended without the words,
-// ends the wait.
+// Wait for a check on `like`'s device: the longest segment of its first array
+// (0 unless CSR offsets), or -1 when a value is bad.  Polls the words, and the
+// stream every 100 ms (a query puts a marker into it), so that an error there,
+// or a stream that ended without the words, ends the wait.
 int64_t maxsim_check_wait(Tensor status, Tensor like) {
-  const int64_t words = status.numel() - 1;
+  const int64_t words = status.numel() - 2;
+  TORCH_CHECK(status.device().is_cpu() && status.scalar_type() == at::kLong &&
+                  status.is_contiguous() && words >= 1,
+              "status must be the result of a layout check");
   const int64_t* w = status.data_ptr<int64_t>();
+  TORCH_CHECK(w[words + 1] == check_tag(w, words),
+              "status must be the result of a layout check");
+  TORCH_CHECK(like.device().is_cuda(), "like must be a HIP (torch 'cuda') tensor");
   const hipStream_t stream = reinterpret_cast<hipStream_t>(static_cast<intptr_t>(w[words]));
   c10::hip::HIPGuardMasqueradingAsCUDA guard(like.device());
   int64_t longest = 0;
