@@ -8,6 +8,7 @@
 // with the caching allocator and calls the C ABI on the current HIP stream.
 // The C ABI itself never allocates.
 #include <ATen/ATen.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
@@ -81,11 +82,12 @@ int64_t check_tag(const int64_t* w, int64_t words) {
 
 // Queue the check of a call's index arrays on the current stream, ahead of
 // the call's kernels; the words of the result are for check_wait(), the last
-// two are the stream and a tag that only these results have.  They are pinned
-// memory that the kernel writes: every begin is followed by a wait.  (On a
-// stream of its own, behind an event, the check gained nothing for the largest
-// calls either, whose workgroups leave it no room: 256 x 1000 candidates 1570
-// against 1565 us.)
+// two are the stream and a tag that only these results have.  The words are
+// pinned memory that the kernel writes: freed before it has (a result dropped
+// without a wait, an interrupt between the two), they go back to the allocator
+// behind an event on the stream.  (On a stream of its own, behind an event, the
+// check gained nothing for the largest calls either, whose workgroups leave it
+// no room: 256 x 1000 candidates 1570 against 1565 us.)
 Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) {
   std::vector<Tensor> held;
   maxsim_check_array arrays[MAXSIM_CHECK_ARRAYS];
@@ -106,15 +108,24 @@ Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) 
   const Tensor& first = held.front();
   c10::hip::HIPGuardMasqueradingAsCUDA guard(first.device());
   const int words = maxsim_internal_check_words(arrays, n);
-  Tensor status =
+  Tensor pinned =
       at::empty({words + 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-  int64_t* w = status.data_ptr<int64_t>();
+  int64_t* w = pinned.data_ptr<int64_t>();
   for (int i = 0; i < words; ++i) w[i] = 0;
-  void* stream = current_stream(first);
+  const auto s = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(first.device().index());
+  void* stream = reinterpret_cast<void*>(s.stream());
   w[words] = reinterpret_cast<intptr_t>(stream);
   w[words + 1] = check_tag(w, words);
   check_status(maxsim_internal_check_layout(arrays, n, reinterpret_cast<uint64_t*>(w), stream));
-  return status;
+  auto release = [pinned, s = s.unwrap(), words](void* p) {
+    const int64_t* v = static_cast<const int64_t*>(p);
+    for (int i = 0; i < words; ++i) {
+      if (__atomic_load_n(v + i, __ATOMIC_ACQUIRE) & 1) continue;
+      at::getHostAllocator(at::kCUDA)->record_event(p, pinned.storage().data_ptr().get_context(), s);
+      break;
+    }
+  };
+  return at::from_blob(w, {words + 2}, std::move(release), at::TensorOptions().dtype(at::kLong));
 }
 
 Tensor maxsim_check_padded(Tensor query_lengths, Tensor doc_lengths, int64_t Lq, int64_t Ld) {

@@ -105,3 +105,25 @@ def test_check_waits_when_the_launch_raises():
         with pytest.raises(ValueError, match="doc_lengths"):
             maxsim_amd.score_candidates_padded(q, d, ql, bad)
         maxsim_amd.score_candidates_padded(q, d, ql, dl)
+
+
+def test_dropped_check_keeps_its_words_until_it_has_run():
+    """A check's result dropped while the check still waits in the stream: its
+    pinned words are not handed out again before the check has written them."""
+    n = 4096
+    off = torch.arange(n + 1, dtype=torch.int32, device=DEVICE)
+    a = torch.randn(4096, 4096, device=DEVICE)
+    torch.cuda.synchronize()
+    for _ in range(20):  # tens of milliseconds of work ahead of the check
+        a = (a @ a).clamp_(-1, 1)
+    busy = torch.cuda.Event()
+    busy.record()
+    status = ops.maxsim_check_contrastive(off, n, None)
+    at = status.data_ptr()
+    del status
+    others = [torch.zeros(m, dtype=torch.int64).pin_memory() for m in (3, 4, 5, 6, 7, 8, 16)
+              for _ in range(8)]
+    assert not busy.query(), "the work ahead ended too early for the test to say anything"
+    assert at not in {t.data_ptr() for t in others}
+    torch.cuda.synchronize()
+    assert not any(bool(t.any()) for t in others)
