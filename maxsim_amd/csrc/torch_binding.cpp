@@ -94,8 +94,19 @@ Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) 
   TORCH_CHECK(!checks.empty() && checks.size() <= MAXSIM_CHECK_ARRAYS, "layout check: arrays");
   int n = 0;
   const at::Device device = std::get<0>(checks.front()).device();
+  TORCH_CHECK(device.is_cuda(), "index tensors must be on one HIP (torch 'cuda') device; got ",
+              device);
+  const auto s = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index());
+  // A graph would keep the address of the words and write them on every
+  // replay; and the host cannot wait for a kernel that is only recorded.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const hipError_t asked = hipStreamIsCapturing(s.stream(), &capture);
+  if (asked != hipSuccess) (void)hipGetLastError();
+  TORCH_CHECK(asked == hipSuccess && capture == hipStreamCaptureStatusNone,
+              "maxsim_amd: the checks of offsets, ids and lengths cannot run while the stream is "
+              "captured; turn them off around the capture (set_host_checks(False))");
   for (const auto& [t, kind, limit] : checks) {
-    TORCH_CHECK(t.device().is_cuda() && t.device() == device,
+    TORCH_CHECK(t.device() == device,
                 "index tensors must be on one HIP (torch 'cuda') device; got ", device, " and ",
                 t.device());
     TORCH_CHECK(t.scalar_type() == at::kInt || t.scalar_type() == at::kLong,
@@ -112,7 +123,6 @@ Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) 
       at::empty({words + 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   int64_t* w = pinned.data_ptr<int64_t>();
   for (int i = 0; i < words; ++i) w[i] = 0;
-  const auto s = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(first.device().index());
   void* stream = reinterpret_cast<void*>(s.stream());
   w[words] = reinterpret_cast<intptr_t>(stream);
   w[words + 1] = check_tag(w, words);

@@ -107,6 +107,24 @@ def test_check_waits_when_the_launch_raises():
         maxsim_amd.score_candidates_padded(q, d, ql, dl)
 
 
+def test_check_is_refused_under_capture():
+    """With the checks on, a call inside a graph capture raises before anything
+    is recorded; the capture, later calls and a capture without the checks are
+    not affected."""
+    q, d, ql, dl = make_padded(2, 3, 4, 8, 16, torch.float32, seed=5)
+    want = maxsim_amd.score_candidates_padded(q, d, ql, dl)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    doubled = torch.empty_like(want)
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captured"):
+            maxsim_amd.score_candidates_padded(q, d, ql, dl)
+        torch.add(want, want, out=doubled)
+    graph.replay()
+    assert torch.equal(doubled, 2 * want)
+    assert torch.equal(maxsim_amd.score_candidates_padded(q, d, ql, dl), want)
+
+
 def test_dropped_check_keeps_its_words_until_it_has_run():
     """A check's result dropped while the check still waits in the stream: its
     pinned words are not handed out again before the check has written them."""
