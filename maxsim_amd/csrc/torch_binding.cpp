@@ -799,6 +799,14 @@ TORCH_LIBRARY(maxsim_amd, m) {
         "Tensor documents, Tensor document_offsets, Tensor argmax) -> (Tensor, Tensor)");
 }
 
+// torch.jit.trace leaves the checks out of the graph, as it did when they were
+// copies to the host: it cannot record an operator that returns a number.
+TORCH_LIBRARY_IMPL(maxsim_amd, Tracer, m) {
+  for (const char* name : {"maxsim_check_padded", "maxsim_check_packed",
+                           "maxsim_check_contrastive", "maxsim_check_wait"})
+    m.impl(name, torch::CppFunction::makeFallthrough());
+}
+
 TORCH_LIBRARY_IMPL(maxsim_amd, CUDA, m) {
   m.impl("maxsim_forward", &maxsim_forward);
   m.impl("maxsim_padded_forward", &maxsim_padded_forward);

@@ -10,7 +10,7 @@ import torch
 import maxsim_amd
 from maxsim_amd._ops import ops
 
-from ._helpers import DEVICE, make_packed, make_padded
+from ._helpers import DEVICE, make_contrastive, make_packed, make_padded
 
 pytestmark = pytest.mark.gpu
 
@@ -145,3 +145,26 @@ def test_dropped_check_keeps_its_words_until_it_has_run():
     assert at not in {t.data_ptr() for t in others}
     torch.cuda.synchronize()
     assert not any(bool(t.any()) for t in others)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")
+def test_jit_trace_of_the_checked_functions():
+    """torch.jit.trace records the scoring operators with the host checks on
+    (the checks themselves stay out of the graph); the traced function scores
+    other inputs of the same shapes."""
+    q, d, off = make_contrastive(3, 8, 32, [5, 9, 7], torch.float32, seed=1)
+    pq, pd, ql, dl = make_padded(2, 3, 4, 8, 16, torch.float32, seed=2)
+    packed = make_packed(3, 4, 6, 32, (4, 12), (5, 20), torch.float32, seed=3)
+    for fn, args in [(maxsim_amd.score_contrastive, (q, d, off)),
+                     (maxsim_amd.score_contrastive_with_argmax, (q, d, off)),
+                     (maxsim_amd.score_candidates_padded, (pq, pd, ql, dl)),
+                     (maxsim_amd.score_pairs_packed, tuple(packed))]:
+        traced = torch.jit.trace(fn, args)
+        assert "maxsim_check" not in str(traced.graph)
+        other = (torch.flip(args[0], (-1,)), *args[1:])
+        for a in (args, other):
+            got, want = traced(*a), fn(*a)
+            for g, w in zip(got if isinstance(got, tuple) else (got,),
+                            want if isinstance(want, tuple) else (want,)):
+                assert torch.equal(g, w)
