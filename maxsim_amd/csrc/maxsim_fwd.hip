@@ -2148,9 +2148,9 @@ struct ContrastiveRoute {
   size_t ws = 0;        // ... of this many bytes (0: not worth it)
 };
 
-// A copy of the documents beyond this is not made (the pair kernels read
-// them in place).
-constexpr size_t kMaxDocCopy = (size_t)4 << 30;
+// A workspace (query fragments and copied documents) beyond this is not asked
+// for (the pair kernels read the rows in place).
+constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // 16-bit rows that could be used in place have the queries' fragments put in
 // order (one launch more, about 3 us) from this many operations: 7e9 at dim 96
 // ran 33.1 us without and 36.8 us with it, 2e10 at dim 256 101.9 and 83.6 us;
@@ -2191,7 +2191,7 @@ static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int
                      2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps))
     return r;
   r.ws = kloop_workspace_bytes(dtype, nq, nblk, total_d, dim, r.copy_d);
-  if (r.ws > kMaxDocCopy) r.ws = 0;
+  if (r.ws > kMaxWorkspace) r.ws = 0;
   return r;
 }
 

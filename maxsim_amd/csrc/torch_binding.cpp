@@ -530,14 +530,20 @@ Contrastive prep_contrastive(Tensor queries, Tensor documents, Tensor document_o
 }
 
 // The forward with the workspace its kernel can use, if any (from torch's
-// allocator, on the current stream like the launches that use it).
+// allocator, on the current stream like the launches that use it).  It is up
+// to a copy of the documents: where the device has no room for it, the kernels
+// without one give the same bits.
 void run_contrastive_forward(const Contrastive& c, int64_t nq, int64_t lq, int64_t nb,
                              const Tensor& scores, int32_t* argmax) {
   const maxsim_dtype dt = to_dtype(c.q);
-  const size_t bytes = maxsim_internal_contrastive_forward_workspace(
+  size_t bytes = maxsim_internal_contrastive_forward_workspace(
       dt, c.q.data_ptr(), nq, lq, c.d.data_ptr(), c.d.size(0), nb, c.q.size(2));
   Tensor ws;
-  if (bytes > 0) ws = at::empty({(int64_t)bytes}, c.q.options().dtype(at::kByte));
+  try {
+    if (bytes > 0) ws = at::empty({(int64_t)bytes}, c.q.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    bytes = 0;
+  }
   check_status(maxsim_internal_contrastive_forward(
       dt, c.q.data_ptr(), nq, lq, c.d.data_ptr(), c.d.size(0), c.off.data_ptr<int32_t>(), nb,
       c.q.size(2), scores.data_ptr<float>(), argmax, bytes > 0 ? ws.data_ptr() : nullptr, bytes,

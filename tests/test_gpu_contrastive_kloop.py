@@ -117,3 +117,23 @@ def test_kloop_nan_and_infinity():
     s, a = _without_workspace(q, d, off)
     torch.testing.assert_close(scores, s, rtol=0, atol=0, equal_nan=True)
     assert torch.equal(a, argmax)
+
+
+def test_kloop_without_room_for_the_workspace():
+    """Where the device has no room for the workspace, the forward runs on the
+    kernels that need none, with the same bits."""
+    torch.cuda.empty_cache()  # the inputs in segments of their own, with nothing free in them
+    q, d, off = make_contrastive(16, 32, 100, [130] * 10000, BF16, seed=9, unit=True)
+    scores, argmax = maxsim_amd.score_contrastive_with_argmax(q, d, off)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info(q.device)[1]
+    torch.cuda.set_per_process_memory_fraction(
+        (torch.cuda.memory_reserved() + (64 << 20)) / total)  # the copy takes 290 MB
+    try:
+        got, got_am = maxsim_amd.score_contrastive_with_argmax(q, d, off)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(128 << 20, dtype=torch.uint8, device=q.device)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, scores) and torch.equal(got_am, argmax)
