@@ -33,6 +33,7 @@
 #include <string>
 #include <type_traits>
 #include <cstdio>
+#include <cmath>
 #include <cstdarg>
 
 #include "maxsim_common.h"
@@ -2079,7 +2080,7 @@ constexpr int tiled_nbw() {
 template <typename T, int KS>
 static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   if constexpr (4 * 32 * KS * 16 * T::bytes + kDocTableBytes > 64 * 1024) {
-    return;  // excluded by tiled_supported(): four buffers would exceed 64 KB
+    return;  // excluded by tiled_blocks(): four buffers would exceed 64 KB
   } else {
   constexpr int NBW = tiled_nbw<T, KS>();
   using G = TileGeom<T, KS>;
@@ -2111,22 +2112,19 @@ static void launch_tiled_ks(TiledArgs a, hipStream_t st) {
   }
 }
 
+// Query blocks of a wave of the tiled kernel, 0 for rows that it does not take:
+// four LDS tile buffers of 32 rows x ks*16 elements (plus the document list)
+// must fit in 64 KB.
 template <typename T>
-static bool tiled_supported(int dim, int lq) {
+static int tiled_blocks(int dim) {
   const int ks = ks_for_dim(dim);
-  // four LDS tile buffers of 32 rows x ks*16 elements (plus the document
-  // list) must fit in 64 KB
-  if (4 * 32 * ks * 16 * T::bytes + kDocTableBytes > 64 * 1024) return false;
-  int nbw = 1;
+  if (4 * 32 * ks * 16 * T::bytes + kDocTableBytes > 64 * 1024) return 0;
   switch (ks) {
-    case 2: nbw = tiled_nbw<T, 2>(); break;
-    case 4: nbw = tiled_nbw<T, 4>(); break;
-    case 8: nbw = tiled_nbw<T, 8>(); break;
-    default: nbw = tiled_nbw<T, 16>(); break;
+    case 2: return tiled_nbw<T, 2>();
+    case 4: return tiled_nbw<T, 4>();
+    case 8: return tiled_nbw<T, 8>();
+    default: return tiled_nbw<T, 16>();
   }
-  // a query's blocks fit one workgroup
-  const int nblk = (lq + kTileCols - 1) / kTileCols;
-  return nblk <= kTiledWaves * nbw;
 }
 
 template <typename T>
@@ -2154,24 +2152,55 @@ constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // 16-bit rows that could be used in place have the queries' fragments put in
 // order (one launch more, about 3 us) from this many operations: 7e9 at dim 96
 // ran 33.1 us without and 36.8 us with it, 2e10 at dim 256 101.9 and 83.6 us;
+// wider rows always;
 // fp32, bound by its MFMAs, gained nothing
 constexpr double kFragMinOps = 1e10;
 
-static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int64_t nq,
-                                          int64_t lq, const void* d, int64_t total_d, int64_t nb,
-                                          int64_t dim) {
-  ContrastiveRoute r;
-  const bool ptrs = aligned16(q) && aligned16(d);
-  if (dim == ks_for_dim((int)dim) * kChunk && ptrs) {
-    switch (dtype) {
-      case MAXSIM_BFLOAT16: r.tiled = tiled_supported<BF16>((int)dim, (int)lq); break;
-      case MAXSIM_FLOAT16: r.tiled = tiled_supported<F16>((int)dim, (int)lq); break;
-      default: r.tiled = tiled_supported<F32>((int)dim, (int)lq); break;
-    }
+// A workgroup of the tiled or K-loop kernel multiplies all its query blocks
+// (`cap` of them), queries or not.  `slots`: what a batch of nq queries of nblk
+// blocks costs in blocks.
+static int64_t block_slots(int64_t nq, int64_t nblk, int64_t cap) {
+  const int64_t qpg = cap / nblk;
+  return (nq + qpg - 1) / qpg * cap;
+}
+
+// Whether queries of more blocks than a wave holds go to the tiled kernel, or
+// to the pair kernels.  With at least a pair per SIMD both are bound by their
+// throughput, and a slot of the tiled kernel costs `slot` of a pair kernel's
+// block.  With fewer pairs the pair kernels take a workgroup per pair, in turn
+// for its blocks; the tiled kernel's time is a document's in one workgroup,
+// that of `serial` such turns.  Pair / tiled kernels, documents of 40-512 rows
+// (1000-4000 for four), us: fp32 dim 64, 96 tokens: 1 query x 4 documents 126 /
+// 482, x 256 25 / 74, x 1000 76 / 203, 10 of 77 x 1000 456 / 353, 9 of 250 x
+// 500 580 / 378; bf16 dim 64: 1 of 77 x 1000 27 / 39, 3 x 1000 51 / 39, 1 of 128
+// x 4000 34 / 63, 20 of 96 x 500 136 / 53; bf16 dim 128: 1 of 77 x 4000 49 /
+// 76, 3 129 / 77; fp16 dim 32: 1 of 77 x 256 8 / 12, 5 x 1000 40 / 35.
+static bool long_queries_tiled(maxsim_dtype dtype, int64_t dim, int64_t nq, int64_t nblk,
+                               int64_t nb, int64_t cap) {
+  const bool f32 = dtype == MAXSIM_FLOAT32;
+  const bool narrow = !f32 && dim <= 32;
+  const double slot = f32 ? 0.74 : narrow ? 0.875 : dim <= 64 ? 0.5 : 0.3125;
+  const double serial = f32 ? 9.5 : narrow ? 7.0 : dim <= 64 ? 3.9 : 2.75;
+  const int64_t slots = block_slots(nq, nblk, cap);
+  const double pairs = (double)nq * (double)nb / device_cus();  // per CU
+  const double wgs = (double)(slots / cap) * (double)nb / device_cus();
+  if (pairs >= 4.0) {
+    const double rounds = std::ceil(pairs / 4.0);  // of a wave per pair
+    return (double)(nq * nblk) * rounds / (pairs / 4.0) > slot * (double)slots;
   }
-  if (r.tiled) return r;
-  const int64_t nblk = (lq + kTileCols - 1) / kTileCols;
-  if (!kloop_supported(dtype, dim, nblk)) return r;
+  // workgroups beyond one per CU share it
+  const double pair_turns = std::max(1.0, 0.5 + 0.5 * pairs);
+  const double tiled_turns = std::max(1.0, narrow ? wgs : 0.5 + 0.5 * wgs);
+  return (double)nblk * pair_turns > serial * tiled_turns;
+}
+
+// Whether rows that the tiled kernel does not take go to the K-loop kernel, or
+// to the pair kernels.
+static bool kloop_pays(maxsim_dtype dtype, int64_t dim, bool vec, bool copy_d, int64_t nq,
+                       int64_t nblk, int64_t nb) {
+  const bool f32 = dtype == MAXSIM_FLOAT32;
+  const int64_t cus = device_cus();
+  const int64_t work = nq * nb * nblk;
   // Few pairs: a workgroup (or wave) per pair, where the K-loop kernel's time
   // is its longest document's, in one workgroup.  Documents of 47-428 rows,
   // pair / K-loop kernels: bf16 dim 256, 256 pairs 11 / 27 us, 512 19 / 28,
@@ -2179,16 +2208,57 @@ static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int
   // 992 pairs 52 / 72 us, 2025 73 / 87, 2400 of 300 queries 86 / 131, 3600 129
   // / 104, with four blocks per query 256 pairs 55 / 72; fp32 dim 384, 32 pairs
   // 123 / 199; bf16 dim 384, 32 pairs 48 / 36.
-  const int64_t cus = device_cus();
-  if (dtype == MAXSIM_FLOAT32
-          ? nblk <= 4 && nq * nb * nblk < 12 * cus
-          : dim <= kMaxRegDim && nblk <= 2 && nq * nb * nblk < 3 * cus)
-    return r;
+  if (f32 ? nblk <= 4 && work < 12 * cus : dim <= kMaxRegDim && nblk <= 2 && work < 3 * cus)
+    return false;
+  // Workgroups that queries do not fill: a slot of the K-loop kernel against a
+  // block of the pair kernels, which are slower the wider or less aligned the
+  // rows, and the documents' copy in slots.  4000 documents of 47-300 rows,
+  // queries of one block, pair / K-loop kernels, us: fp32 dim 128, 1 query 115 /
+  // 463, 4 371 / 470, 9 698 / 838, 16 1191 / 854; fp32 dim 72, 2 214 / 388, 6
+  // 540 / 391; fp32 dim 384, 1 519 / 1323, 4 1719 / 1339; bf16 dim 256, 1 74 /
+  // 132, 4 243 / 137; bf16 dim 100 (copied), 1 36 / 128, 6 155 / 129; bf16 dim
+  // 300 (copied), 1 246 / 314, 2 462 / 317; bf16 dim 768, 1 498 / 333.
+  double slot, copy;
+  if (f32) {
+    if (nblk > 4 && nq * nb < 4 * cus) return true;  // a pair's blocks in turn
+    slot = dim > kMaxRegDim ? 0.375
+           : vec            ? (dim > 128 ? 0.7 : 0.75)
+                            : (dim > 128 ? 0.25 : 0.5);
+    copy = 2.0;
+  } else {
+    if (dim > kMaxRegDim && work < 3 * cus) return true;  // the wide pair kernel's latency
+    slot = dim > kMaxRegDim ? 0.1 : !vec && dim > 128 ? 0.25 : 0.35;
+    copy = dim > kMaxRegDim ? 6.0 : dim > 128 ? 3.5 : 5.0;
+  }
+  return (double)(nq * nblk) >
+         slot * ((double)block_slots(nq, nblk, kKloopBlocks) + (copy_d ? copy : 0.0));
+}
+
+static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int64_t nq,
+                                          int64_t lq, const void* d, int64_t total_d, int64_t nb,
+                                          int64_t dim) {
+  ContrastiveRoute r;
+  const bool ptrs = aligned16(q) && aligned16(d);
+  const bool vec = dim == ks_for_dim((int)dim) * kChunk && ptrs;
+  const int64_t nblk = (lq + kTileCols - 1) / kTileCols;
+  if (vec) {
+    const int nbw = dtype == MAXSIM_BFLOAT16  ? tiled_blocks<BF16>((int)dim)
+                    : dtype == MAXSIM_FLOAT16 ? tiled_blocks<F16>((int)dim)
+                                              : tiled_blocks<F32>((int)dim);
+    const int64_t cap = (int64_t)kTiledWaves * nbw;
+    if (nblk <= cap) {
+      r.tiled = nblk <= nbw || long_queries_tiled(dtype, dim, nq, nblk, nb, cap);
+      return r;
+    }
+  }
+  if (!kloop_supported(dtype, dim, nblk)) return r;
+  const bool copy_d = !(dim % kChunk == 0 && aligned16(d));
+  if (!kloop_pays(dtype, dim, vec, copy_d, nq, nblk, nb)) return r;
   r.kloop = true;
   r.in_place = dim % kChunk == 0 && ptrs;
-  r.copy_d = !(dim % kChunk == 0 && aligned16(d));
-  if (r.in_place && (dtype == MAXSIM_FLOAT32 ||
-                     2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps))
+  r.copy_d = copy_d;
+  if (r.in_place && (dtype == MAXSIM_FLOAT32 || (dim <= kMaxRegDim &&
+                     2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps)))
     return r;
   r.ws = kloop_workspace_bytes(dtype, nq, nblk, total_d, dim, r.copy_d);
   if (r.ws > kMaxWorkspace) r.ws = 0;
@@ -2262,6 +2332,14 @@ size_t maxsim_internal_contrastive_forward_workspace(maxsim_dtype dtype, const v
     return 0;
   return contrastive_route(dtype, queries, num_queries, Lq, documents, total_d_tokens,
                            num_documents, dim).ws;
+}
+
+int maxsim_internal_contrastive_route(maxsim_dtype dtype, const void* queries, int64_t num_queries,
+                                      int64_t Lq, const void* documents, int64_t total_d_tokens,
+                                      int64_t num_documents, int64_t dim) {
+  const ContrastiveRoute r = contrastive_route(dtype, queries, num_queries, Lq, documents,
+                                               total_d_tokens, num_documents, dim);
+  return r.tiled ? 1 : !r.kloop ? 0 : r.ws > 0 ? 3 : r.in_place ? 2 : 0;
 }
 
 int maxsim_internal_contrastive_forward(

@@ -17,6 +17,12 @@ size_t maxsim_internal_contrastive_forward_workspace(maxsim_dtype dtype, const v
                                                      const void* documents, int64_t total_d_tokens,
                                                      int64_t num_documents, int64_t dim);
 
+/* The kernel of that forward: 0 a pair kernel, 1 the tiled one, 2 the K-loop
+ * kernel on the rows in place, 3 the K-loop kernel with the workspace. */
+int maxsim_internal_contrastive_route(maxsim_dtype dtype, const void* queries, int64_t num_queries,
+                                      int64_t Lq, const void* documents, int64_t total_d_tokens,
+                                      int64_t num_documents, int64_t dim);
+
 /* maxsim_amd_contrastive_forward_with_argmax (argmax may be NULL) with a
  * workspace; a NULL, misaligned or smaller one gives that entry point's
  * result without it.  Same results, bit for bit, either way. */

@@ -51,6 +51,7 @@ constexpr int kKlTilePieces = kTileRows * kKlPieces;
 constexpr int kKlUnitPieces = kKlTiles * kKlTilePieces;
 constexpr int kKlMaxDocs = 1024;              // document list per workgroup
 static_assert(kKlTiles == kKlWaves, "wave w loads tile w");
+static_assert(kKlWaves * kKlBlocks == kKloopBlocks, "as the route counts them");
 
 template <typename T, bool ARGMAX>
 __global__ __launch_bounds__(kKlThreads, 2) void contrastive_kloop_kernel(TiledArgs a) {

@@ -220,6 +220,7 @@ inline int64_t chunks_for_rounds(int64_t n_qg, int64_t tiles, int64_t resident) 
 // first brings the queries, and the documents if copy_d, into the kernel's
 // layout (and points `a` at them).  `a` comes without the launch's own fields
 // (qpg, n_qg, n_dc).
+constexpr int kKloopBlocks = 8;  // query blocks of a workgroup
 bool kloop_supported(maxsim_dtype dtype, int64_t dim, int64_t nblk);
 size_t kloop_workspace_bytes(maxsim_dtype dtype, int64_t nq, int64_t nblk, int64_t total_d,
                              int64_t dim, bool copy_d);
