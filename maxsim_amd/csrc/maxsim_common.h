@@ -155,8 +155,8 @@ __device__ __forceinline__ Frag<T> load_frag(const typename T::storage* row,
 
 // A row's KS chunks (16 elements each, this lane's halves at 8 * h) for the
 // kernels that hold a whole row, by a constant of the launch: aligned whole
-// fragments; rows of at least 8 elements that start anywhere; shorter ones,
-// element by element.  Chunks past the embedding dimension are neither loaded
+// fragments; rows of at least 8 elements that start anywhere; shorter ones (and
+// fp32 ones of 129 elements and more, for their registers), element by element.  Chunks past the embedding dimension are neither loaded
 // nor (mma_chunks) multiplied.  (Its own constant for the short rows: their
 // loads' many branches would spill scalar registers in every kernel.)  Rows
 // of widths such as 96, 100 or 300 were read element by element before:

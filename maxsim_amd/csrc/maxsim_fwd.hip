@@ -1804,6 +1804,17 @@ static bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
 
+// fp32 rows of 129 to 256 elements that are not whole aligned fragments are
+// loaded element by element: in whole fragments (kRowAny) the two tiles and the
+// query block in registers spill 360-570 vector registers.  Padded, 32 x 100
+// candidates, 300 x 24 tokens, in whole fragments / element by element, us: dim
+// 130 384 / 225, dim 200 471 / 344, dim 255 604 / 296.  (The kernels with up to
+// 50 spilled ones, fp32 rows of 65 to 128 and 16-bit ones of 129 to 256 with two
+// query blocks, gain all the same: 16 x 100 candidates, 64 query tokens, fp32
+// dim 96 111 / 73, bf16 dim 200 181 / 63 element by element / in fragments.)
+template <typename T, int KS>
+constexpr bool kAnySpills = T::bytes == 4 && KS == 16;
+
 template <typename T, int KS, int QB, int LOAD>
 static void launch_pair_load(const FwdArgs& a, int ppw, dim3 grid, hipStream_t st) {
   hipLaunchKernelGGL((a.argmax ? pair_kernel<T, KS, QB, true, LOAD>
@@ -1815,9 +1826,13 @@ template <typename T, int KS, int QB>
 static void launch_pair_qb(const FwdArgs& a, int ppw, bool vec, dim3 grid,
                            hipStream_t st) {
   if (vec) return launch_pair_load<T, KS, QB, kRowVec>(a, ppw, grid, st);
-  if constexpr (KS == 2)
-    if (a.dim < 8) return launch_pair_load<T, KS, QB, kRowShort>(a, ppw, grid, st);
-  launch_pair_load<T, KS, QB, kRowAny>(a, ppw, grid, st);
+  if constexpr (kAnySpills<T, KS>) {
+    launch_pair_load<T, KS, QB, kRowShort>(a, ppw, grid, st);
+  } else {
+    if constexpr (KS == 2)
+      if (a.dim < 8) return launch_pair_load<T, KS, QB, kRowShort>(a, ppw, grid, st);
+    launch_pair_load<T, KS, QB, kRowAny>(a, ppw, grid, st);
+  }
 }
 
 template <typename T, int KS>
@@ -1854,9 +1869,13 @@ static void launch_split_load(const FwdArgs& a, hipStream_t st) {
 template <typename T, int KS>
 static void launch_split_ks(const FwdArgs& a, bool vec, hipStream_t st) {
   if (vec) return launch_split_load<T, KS, kRowVec>(a, st);
-  if constexpr (KS == 2)
-    if (a.dim < 8) return launch_split_load<T, KS, kRowShort>(a, st);
-  launch_split_load<T, KS, kRowAny>(a, st);
+  if constexpr (kAnySpills<T, KS>) {
+    launch_split_load<T, KS, kRowShort>(a, st);
+  } else {
+    if constexpr (KS == 2)
+      if (a.dim < 8) return launch_split_load<T, KS, kRowShort>(a, st);
+    launch_split_load<T, KS, kRowAny>(a, st);
+  }
 }
 
 template <typename T>
