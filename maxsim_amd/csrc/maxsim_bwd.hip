@@ -815,6 +815,15 @@ constexpr int kDdBatch = 8;      // bucket entries gathered per step
 constexpr int kDdBlock = 32;     // bucket entries per block sum
 constexpr int kDdSortBatch = 8;  // argmax loads in flight per thread while sorting
 
+// Waves per SIMD that dd_contrastive_kernel is compiled for, aligned rows of one
+// slice per lane: four, two workgroups per CU.  Left to itself the compiler
+// takes 129 registers for fp32, one too many: 300 x 300 documents of 20-400
+// rows, dim 200, 253 -> 216 us.  (Not with dq in the launch, where the second
+// workgroup gets in dq's way: whole backward, 30 queries of 20 tokens x 150
+// documents, dim 200, 36 us at three waves, 47 at four.)
+template <bool VEC, int NS>
+constexpr int kDdMinWaves = VEC && NS == 1 ? 4 : 1;
+
 // x / d for 0 <= x < 2^24, d >= 1, from a float reciprocal: x is exact in
 // fp32 and the rounded product is within one of the quotient (exact for
 // d <= 2), so one remainder check gives the exact result.  Avoids the
@@ -1046,7 +1055,8 @@ __device__ __forceinline__ void dd_contrastive_document(const DdArgs& a, unsigne
 }
 
 template <typename T, bool VEC, int NS, typename O>
-__global__ __launch_bounds__(kDdThreads) void dd_contrastive_kernel(DdArgs a) {
+__global__ __launch_bounds__(kDdThreads, (kDdMinWaves<VEC, NS>)) void dd_contrastive_kernel(
+    DdArgs a) {
   dd_contrastive_document<T, VEC, NS, O>(a, blockIdx.x);
 }
 

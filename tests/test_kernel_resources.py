@@ -63,3 +63,10 @@ def test_no_kernel_spills_its_operands(kernels):
     spilled = {n: k[".vgpr_spill_count"] for n, k in kernels.items()
                if k[".vgpr_spill_count"] > 50}
     assert not spilled, spilled
+
+
+def test_contrastive_dd_two_workgroups_per_cu(kernels):
+    # 512 threads are two waves per SIMD: four waves in 512 registers
+    of = {n: k[".vgpr_count"] for n, k in kernels.items()
+          if n.startswith("dd_contrastive_kernel<") and ", true, 1, " in n}
+    assert len(of) == 5 and max(of.values()) <= 128, of
