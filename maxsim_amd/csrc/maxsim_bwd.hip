@@ -334,19 +334,40 @@ constexpr int kDqBatch = 4;
 constexpr int kDqSplitMaxDim = 2048;  // 8 * 256 slices: one row per workgroup at most
 constexpr int kDqTable = 2048;  // (row, document) pairs staged per chunk
 
+// PACED (fp32): the gathers are held back.  An XCD's waves walk the same
+// documents side by side, and the L2 serves them only as long as they stay
+// together: with several loads of 32 bytes per lane in flight, or eight waves
+// per SIMD, they drift apart and each fetches its rows anew.  So each load is
+// waited for before the next, and the table takes the LDS that leaves six
+// workgroups to a CU.  Whole backward, four loads in flight / paced, documents
+// of 20-400 rows, us: dim 256, 512 x 512 1294 / 1022, 64 x 600 219 / 196; dim
+// 384, 300 x 300 660 / 494; dim 768, 40 x 1500 1353 / 1146; but dim 64, 64 x 600
+// 74 / 87 and dim 128, 40 x 1500 184 / 215, whose rows are few and short.
+constexpr int kDqPacedTable = 3328;
+static_assert(6 * kDqPacedTable * 8 <= 160 * 1024 && 7 * kDqPacedTable * 8 > 160 * 1024,
+              "six workgroups per CU");
+static bool dq_paced(int64_t rows, int64_t dim) {
+  return dim > 128 || rows * dim * 4 > (int64_t)(4 << 20);
+}
+// Waits for a loaded fragment here instead of where it is used.
+__device__ __forceinline__ void wait_frag(Frag<F32>& f) {
+  __asm__ __volatile__("" : "+v"(f.lo.x), "+v"(f.hi.x));
+}
+
 // VEC: 16-byte rows, a template parameter so that a batch's loads need no
 // branch between them (a join there waits for each): bf16, 300 x 300 documents
-// of 20-200 rows, whole backward at dim 768 460 -> 446 us, at dim 300 1985 ->
-// 450 us (rows on any boundary in whole fragments).
-template <typename T, int U, bool VEC>
+// of 20-200 rows, whole backward at dim 300 1985 -> 450 us (rows on any boundary
+// in whole fragments).
+template <typename T, int U, bool VEC, bool PACED>
 __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, float* ws, int rows_per_group) {
   using S = typename T::storage;
-  __shared__ int32_t t_src[kDqTable];  // [document in chunk][row in group]
-  __shared__ float t_w[kDqTable];
+  constexpr int kTable = PACED ? kDqPacedTable : kDqTable;
+  __shared__ int32_t t_src[kTable];  // [document in chunk][row in group]
+  __shared__ float t_w[kTable];
   const int r = blockIdx.x % kXcds;
   const int64_t row0 = (int64_t)(blockIdx.x / kXcds) * rows_per_group;
   const int rpg = rows_per_group;
-  const int chunk = kDqTable / rpg;
+  const int chunk = kTable / rpg;
   const int tid = threadIdx.x;
   const int local = tid / a.nslices;
   const int64_t row = row0 + local;
@@ -395,6 +416,7 @@ __global__ __launch_bounds__(256) void dq_split_kernel(DqArgs a, float* ws, int 
           const int e = (MASKED ? min(bl + u, nc - 1) : bl + u) * rpg + local;
           wt[u] = t_w[e];
           v[u] = load_frag<T>(D + (int64_t)t_src[e] * a.dim, k0, a.dim, VEC);
+          if constexpr (PACED) wait_frag(v[u]);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -2649,9 +2671,19 @@ static void launch_dq_split(const DqArgs& a, bool vec, float* ws, bool vec_reduc
                             bool reduce, hipStream_t st) {
   const int rows_per_group = 256 / a.nslices;  // >= 8: dim <= 256
   const int64_t n_groups = (a.rows + rows_per_group - 1) / rows_per_group;
-  hipLaunchKernelGGL((vec ? dq_split_kernel<T, kDqBatch, true>
-                          : dq_split_kernel<T, kDqBatch, false>),
-                     dim3((unsigned)(n_groups * kXcds)), dim3(256), 0, st, a, ws, rows_per_group);
+  auto kern = vec ? dq_split_kernel<T, kDqBatch, true, false>
+                  : dq_split_kernel<T, kDqBatch, false, false>;
+  if constexpr (T::bytes == 4) {
+    if (vec && dq_paced(a.rows, a.dim)) kern = dq_split_kernel<T, 1, true, true>;
+  } else {
+    // wide 16-bit rows drift apart too (PACED): two loads in flight where there
+    // are many documents.  Whole backward, bf16, four / two: dim 384, 512 x 512
+    // documents 972 / 854 us, dim 768, 64 x 600 489 / 453, 500 x 100 477 / 490;
+    // dim 256, 40 x 1500 235 / 244
+    if (vec && a.dim > 256 && a.nb >= 32 * kXcds) kern = dq_split_kernel<T, 2, true, false>;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)(n_groups * kXcds)), dim3(256), 0, st, a, ws,
+                     rows_per_group);
   if (!reduce) return;  // the dD launch adds the partial sums
   const int64_t n = a.rows * a.dim;
   const int64_t work = vec_reduce ? n / 4 : n;
