@@ -27,6 +27,7 @@
 // are zero-filled and accumulated with hardware fp32 global atomics.
 #include "maxsim_common.h"
 #include "maxsim_host.h"
+#include "maxsim_internal.h"
 
 #include <algorithm>
 #include <mutex>
@@ -3011,6 +3012,20 @@ static int packed_backward_impl(
   return check_launch("grads_packed_kernel");
 }
 
+// Whether dq runs in the dd launch, as far as the documents go (vec: aligned
+// rows; dd_bucket: the bucketing dd).  One launch saves a launch and the shorter kernel's time, but
+// halves the CUs of dq, whose waves walk every document, and with 32-byte
+// gathers that costs it a few ns per document.  Whole backward, fp32, one launch
+// / two, us: dim 64, 8 queries x 64 documents 15 / 20, x 150 46 / 43, x 300 92 /
+// 80, 64 queries x 300 96 / 101; dim 128, 8 x 700 171 / 168, x 2000 727 / 559; dim
+// 256, 8 x 700 193 / 214, x 2000 762 / 680; unaligned rows, dim 300, 8 x 2000 1223
+// / 1744; in bf16 8 x 2000 273 / 322.
+static bool grads_one_launch(maxsim_dtype dtype, bool vec, bool dd_bucket, int64_t rows,
+                             int64_t nb, int64_t dim) {
+  if (dtype != MAXSIM_FLOAT32 || !vec) return true;
+  return nb <= (dd_bucket && dim <= 64 ? std::max<int64_t>(128, rows / 4) : 1024);
+}
+
 static int contrastive_backward_impl(
     maxsim_dtype dtype, maxsim_dtype grad_dtype, const float* dscore, const CeGrad& ce,
     const void* queries, int64_t num_queries, int64_t Lq, const void* documents,
@@ -3206,7 +3221,8 @@ static int contrastive_backward_impl(
       ba.dq_n = num_queries * Lq * dim;
       ba.dq_vec = vec_reduce ? 1 : 0;
     }
-  } else if (nslices <= 256 && off32 && grads_args(qa, da).dq_wgs <= (unsigned)device_cus()) {
+  } else if (nslices <= 256 && off32 && grads_args(qa, da).dq_wgs <= (unsigned)device_cus() &&
+             grads_one_launch(dtype, vec, bucket, qa.rows, num_documents, dim)) {
     // dq in the dd launch, while its workgroups leave most of the chip to
     // dd's.  Whole backward, bf16, one launch / two: 64 x 64 documents at dim
     // 128 (64 workgroups) 21 / 24.5 us, fp32 72 x 72 (72) 29 / 41; at dim 768
@@ -3262,6 +3278,12 @@ int maxsim_amd_contrastive_backward_typed(
                                    documents, total_d_tokens, document_offsets, num_documents,
                                    argmax, dim, dqueries, ddocuments, workspace, workspace_bytes,
                                    stream);
+}
+
+int maxsim_internal_contrastive_grads_one_launch(maxsim_dtype dtype, int vec, int dd_bucket,
+                                                 int64_t rows, int64_t num_documents,
+                                                 int64_t dim) {
+  return grads_one_launch(dtype, vec != 0, dd_bucket != 0, rows, num_documents, dim) ? 1 : 0;
 }
 
 int maxsim_amd_contrastive_ce_backward_typed(

@@ -33,6 +33,12 @@ int maxsim_internal_contrastive_forward(maxsim_dtype dtype, const void* queries,
                                         int32_t* argmax, void* workspace, size_t workspace_bytes,
                                         void* stream);
 
+/* 1 where the contrastive gradients' documents allow both in one launch (vec:
+ * aligned rows; dd_bucket: the bucketing dd kernel takes the batch). */
+int maxsim_internal_contrastive_grads_one_launch(maxsim_dtype dtype, int vec, int dd_bucket,
+                                                 int64_t rows, int64_t num_documents,
+                                                 int64_t dim);
+
 /* One index array of a layout check: CSR offsets (strictly increasing from 0
  * to `limit`), ids in [0, limit) or lengths in [1, limit]; int32 or int64. */
 enum maxsim_check_kind { MAXSIM_CHECK_CSR = 0, MAXSIM_CHECK_IDS = 1, MAXSIM_CHECK_LENGTHS = 2 };

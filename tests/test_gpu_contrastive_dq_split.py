@@ -42,8 +42,8 @@ def test_contrastive_dq_split(dtype, dim, Nq, Lq, Nb):
     dq, _ = ops.maxsim_contrastive_backward(g, q, d, off, am)
     want = torch.zeros(Nq, Lq, dim, dtype=torch.float64, device=DEVICE)
     size = torch.zeros_like(want)
-    for b in range(Nb):
-        rows = d[int(off[b]) + am[:, b].long()].double()
+    for b, start in enumerate(off.tolist()[:-1]):
+        rows = d[start + am[:, b].long()].double()
         term = rows * g[:, b, None, None].double()
         want += term
         size += term.abs()
