@@ -1863,9 +1863,8 @@ __device__ __forceinline__ void dq_padded_rows(const DqArgs& a, int64_t wg) {
 }
 
 // Both padded gradients in one launch: dq's gathers (latency) run under dd's
-// writes (memory bandwidth).  256 queries x 16 candidates of 300 rows, bf16:
-// 82.6 -> 74.9 us (two launches of 18 and 63 us before), 68 x 703 of 66 rows 579
-// -> 474, the same bits.
+// writes (memory bandwidth).  256 queries x 16 candidates of 300 rows, dim 128,
+// bf16: 82.6 -> 74.9 us (two launches of 18 and 63 us before), the same bits.
 // At least six waves per SIMD: dq holds raw fragments, widened as they are added
 // (eight would spill 49 registers in bf16).
 template <typename T, bool VEC, typename O>
@@ -1875,6 +1874,16 @@ __global__ __launch_bounds__(256, (VEC ? 6 : 4)) void grads_padded_kernel(DqArgs
     dq_padded_rows<T, VEC, O>(dq, blockIdx.x);
   else
     dd_padded_rows<T, O>(dd, blockIdx.x - dq_wgs);
+}
+
+// The same in two launches, dd at eight waves per SIMD.
+template <typename T, bool VEC, typename O>
+__global__ __launch_bounds__(256, (VEC ? 6 : 4)) void dq_padded_kernel(DqArgs dq) {
+  dq_padded_rows<T, VEC, O>(dq, blockIdx.x);
+}
+template <typename T, typename O>
+__global__ __launch_bounds__(256) void dd_padded_kernel(PaddedDdArgs dd) {
+  dd_padded_rows<T, O>(dd, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2779,18 +2788,33 @@ static int launch_dd_contrastive(const DdArgs& a, const DqArgs* dq, bool vec, si
 // Largest grid of 256-thread workgroups in one dimension (2^32 - 1 work-items).
 constexpr int64_t kMaxBlocks256 = (int64_t)UINT32_MAX / 256;
 
+// Both padded gradients in one launch, unless dd is long enough to need its
+// waves.  Beyond what the Infinity Cache (256 MB) takes up, two of its forms do
+// not keep the memory busy at dq's registers: 16-bit rows by single elements
+// (dd_padded_rows16) and fp32 ones by whole rows (dd_padded_rows_vec).  One
+// launch / two, us: bf16 dim 768, 256 x 16 candidates of 300 rows 512 / 454, 4 x
+// 16 27 / 33; bf16 dim 100, 256 x 16 112 / 98, 128 x 8 37 / 37; fp32 dim 256, 256
+// x 16 284 / 250, 32 x 100 of 200 149 / 147, dim 128, 64 x 16 of 600 60 / 64; fp32 dim 128, 256 x 64 565 / 493; the
+// other forms: bf16 dim 256, 256 x 64 446 / 521, fp32 dim 768, 64 x 16 of 600 399
+// / 454.
+static bool padded_one_launch(bool out16, bool whole_rows, int64_t dd_bytes) {
+  return dd_bytes <= (int64_t)((out16 ? 192 : 384) << 20) || out16 == whole_rows;
+}
+
 template <typename T, typename O>
 static void launch_padded_o(const DqArgs& q, const PaddedDdArgs& a, bool vec, hipStream_t st) {
   const int64_t dq_wgs = (q.rows * q.nslices * q.csplit + 255) / 256;
   const int64_t dd_wgs = (a.npairs * a.nsplit + 3) / 4;
   // the fp32 output takes the argmax LDS only on the vec_rows path
   const size_t lds = O::bytes == 2 || a.vec_rows ? (size_t)4 * a.am_lds * sizeof(int32_t) : 0;
-  const auto kern = vec ? grads_padded_kernel<T, true, O> : grads_padded_kernel<T, false, O>;
-  if (dq_wgs + dd_wgs <= kMaxBlocks256) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)(dq_wgs + dd_wgs)), dim3(256), lds, st, q, dq_wgs, a);
+  if (dq_wgs + dd_wgs <= kMaxBlocks256 &&
+      padded_one_launch(O::bytes == 2, a.vec_rows, a.npairs * a.ld_max * a.dim * O::bytes)) {
+    hipLaunchKernelGGL((vec ? grads_padded_kernel<T, true, O> : grads_padded_kernel<T, false, O>),
+                       dim3((unsigned)(dq_wgs + dd_wgs)), dim3(256), lds, st, q, dq_wgs, a);
   } else {  // each fits one launch (checked)
-    hipLaunchKernelGGL(kern, dim3((unsigned)dq_wgs), dim3(256), lds, st, q, dq_wgs, a);
-    hipLaunchKernelGGL(kern, dim3((unsigned)dd_wgs), dim3(256), lds, st, q, (int64_t)0, a);
+    hipLaunchKernelGGL((vec ? dq_padded_kernel<T, true, O> : dq_padded_kernel<T, false, O>),
+                       dim3((unsigned)dq_wgs), dim3(256), 0, st, q);
+    hipLaunchKernelGGL((dd_padded_kernel<T, O>), dim3((unsigned)dd_wgs), dim3(256), lds, st, a);
   }
 }
 
@@ -3280,6 +3304,10 @@ int maxsim_amd_contrastive_backward_typed(
                                    stream);
 }
 
+int maxsim_internal_padded_grads_one_launch(int out16, int whole_rows, int64_t dd_bytes) {
+  return padded_one_launch(out16 != 0, whole_rows != 0, dd_bytes) ? 1 : 0;
+}
+
 int maxsim_internal_contrastive_grads_one_launch(maxsim_dtype dtype, int vec, int dd_bucket,
                                                  int64_t rows, int64_t num_documents,
                                                  int64_t dim) {
@@ -3415,7 +3443,7 @@ int maxsim_amd_padded_backward_typed(
   const int64_t am_rest = Lq_max - 64 * kDdAmRegs;
   da.am_lds = (out16 || da.vec_rows) && am_rest > 0 && am_rest <= kDdAmLdsMax ? (int)am_rest : 0;
   MAXSIM_DISPATCH(dtype, launch_padded, qa, da, vec, out16, st);
-  return check_launch("grads_padded_kernel");
+  return check_launch("grads_padded_kernel / dq_padded_kernel, dd_padded_kernel");
 }
 
 int maxsim_amd_padded_backward(

@@ -39,6 +39,10 @@ int maxsim_internal_contrastive_grads_one_launch(maxsim_dtype dtype, int vec, in
                                                  int64_t rows, int64_t num_documents,
                                                  int64_t dim);
 
+/* 1 where both padded gradients are one launch: by the gradients' type, whether
+ * dd writes whole rows per lane group, and dd's bytes. */
+int maxsim_internal_padded_grads_one_launch(int out16, int whole_rows, int64_t dd_bytes);
+
 /* One index array of a layout check: CSR offsets (strictly increasing from 0
  * to `limit`), ids in [0, limit) or lengths in [1, limit]; int32 or int64. */
 enum maxsim_check_kind { MAXSIM_CHECK_CSR = 0, MAXSIM_CHECK_IDS = 1, MAXSIM_CHECK_LENGTHS = 2 };

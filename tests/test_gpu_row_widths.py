@@ -76,3 +76,32 @@ def test_padded_backward_row_widths(B, C, Lq, Ld, dim, dtype):
     assert_close(dd.view(d.shape), dd_ref, **GRAD_TOL[dtype])
     dq16, dd16 = ops.maxsim_padded_backward_typed(*flat)
     assert torch.equal(dq16, dq.to(dtype)) and torch.equal(dd16, dd.to(dtype))
+
+
+@pytest.mark.parametrize("dtype,B,Ld,dim", [
+    (torch.float32, 160, 200, 256),  # whole rows per lane group, fp32
+    (torch.bfloat16, 80, 251, 600),  # single elements, 16 bit
+    (torch.float16, 80, 251, 601),   # rows on any boundary
+])
+def test_padded_backward_two_launches(dtype, B, Ld, dim):
+    """Gradients beyond the size up to which they share a launch, bit for bit
+    those of the batch's halves, which do share one."""
+    C, Lq = 13, 20
+    q, d, ql, dl = make_padded(B, C, Lq, Ld, dim, dtype, seed=dim)
+    limit = (384 if dtype == torch.float32 else 192) << 20
+    assert d.numel() * d.element_size() > limit > d.numel() * d.element_size() // 2
+    gen = torch.Generator().manual_seed(1)
+    a = torch.minimum(torch.randint(0, Ld, (B, C, Lq), generator=gen, dtype=torch.int32).to(q.device),
+                      dl[..., None] - 1)
+    g = torch.randn(B, C, generator=gen).to(q.device)
+
+    def grads(lo, hi):
+        n = hi - lo
+        return ops.maxsim_padded_backward_typed(
+            g[lo:hi].reshape(-1), q[lo:hi].reshape(n * Lq, dim), d[lo:hi].reshape(n * C * Ld, dim),
+            ql[lo:hi], dl[lo:hi].reshape(-1), a[lo:hi].reshape(n * C, Lq), Lq, Ld, C)
+
+    dq, dd = grads(0, B)
+    halves = [grads(0, B // 2), grads(B // 2, B)]
+    assert torch.equal(dq, torch.cat([h[0] for h in halves]))
+    assert torch.equal(dd, torch.cat([h[1] for h in halves]))

@@ -36,3 +36,19 @@ def test_contrastive_gradients(lib, dtype, vec, bucket, rows, nb, dim, one):
     fn = lib.maxsim_internal_contrastive_grads_one_launch
     fn.argtypes = [ctypes.c_int] * 3 + [I64] * 3
     assert fn(dtype, vec, bucket, rows, nb, dim) == one
+
+
+@pytest.mark.parametrize("out16,whole_rows,rows,dim,one", [
+    (1, 0, 4096 * 300, 768, 0),   # 512 us in one launch, 454 in two
+    (1, 0, 4096 * 300, 100, 0),   # 112, 98
+    (1, 0, 1024 * 300, 100, 1),   # 37, 37
+    (1, 0, 64 * 300, 768, 1),     # 27, 33
+    (1, 1, 16384 * 300, 256, 1),  # 446, 521
+    (0, 1, 4096 * 300, 256, 0),   # 284, 250
+    (0, 1, 3200 * 100, 128, 1),   # 39, 44
+    (0, 0, 1024 * 600, 768, 1),   # 399, 454
+])
+def test_padded_gradients(lib, out16, whole_rows, rows, dim, one):
+    fn = lib.maxsim_internal_padded_grads_one_launch
+    fn.argtypes = [ctypes.c_int, ctypes.c_int, I64]
+    assert fn(out16, whole_rows, rows * dim * (2 if out16 else 4)) == one
