@@ -8,6 +8,8 @@ the north-star bounds (1e-5 relative for fp32, 2e-2 for bf16/fp16).
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -129,3 +131,50 @@ def assert_rounded_from(typed: torch.Tensor, ref32: torch.Tensor, mag: torch.Ten
     err = (typed.float() - ref32).abs()
     bound = rel * ref32.abs() + 2.0 ** -16 * mag + atol
     assert bool(torch.all(err <= bound)), float((err - bound).max())
+
+
+# ---- which kernel a contrastive forward takes -------------------------------
+PAIR, TILED, KLOOP, KLOOP_WS = 0, 1, 2, 3
+_TAGS = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+
+
+def contrastive_route(q, d, offsets) -> int:
+    """The kernel of the contrastive forward for these tensors (the host's rule)."""
+    fn = _native().maxsim_internal_contrastive_route
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    fn.argtypes = [ctypes.c_int, ptr, i64, i64, ptr, i64, i64, i64]
+    nq, lq, dim = q.shape
+    return fn(_TAGS[q.dtype], q.data_ptr(), nq, lq, d.data_ptr(), d.shape[0],
+              offsets.numel() - 1, dim)
+
+
+def contrastive_c_abi(q, d, offsets):
+    """Scores and argmax of the C ABI entry point, which takes no workspace."""
+    fn = _native().maxsim_amd_contrastive_forward_with_argmax
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    fn.argtypes = [ctypes.c_int, ptr, i64, i64, ptr, i64, ptr, i64, i64, ptr, ptr, ptr]
+    nq, lq, dim = q.shape
+    nb = offsets.numel() - 1
+    s = torch.empty(nq, nb, device=q.device)
+    a = torch.empty(nq, nb, lq, dtype=torch.int32, device=q.device)
+    assert fn(_TAGS[q.dtype], q.data_ptr(), nq, lq, d.data_ptr(), d.shape[0],
+              offsets.data_ptr(), nb, dim, s.data_ptr(), a.data_ptr(),
+              torch.cuda.current_stream().cuda_stream) == 0
+    return s, a
+
+
+def one_element_off(t):
+    """A copy of ``t`` whose rows start one element past an aligned address."""
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view_as(t).copy_(t)
+
+
+def contrastive_pair_kernels(q, d, offsets):
+    """Scores and argmax of the pair kernels, whatever the shape: rows off any
+    16-byte boundary and no workspace leave nothing else."""
+    return contrastive_c_abi(one_element_off(q), one_element_off(d), offsets)
+
+
+def _native():
+    from maxsim_amd._ops import NATIVE_LIB
+
+    return ctypes.CDLL(str(NATIVE_LIB))

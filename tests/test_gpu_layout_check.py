@@ -1,6 +1,8 @@
 """The device-side layout check behind the Python functions: every array kind
-and index type, one to 64 workgroups, a bad value at either end, on workgroup
-boundaries and in each array, the longest segment, and the reference's errors."""
+and index type, one to 87 workgroups (of at most 128), a bad value at either
+end, on workgroup boundaries and in each array, the longest segment, the
+reference's errors, and the check's result under capture, tracing and when it
+is dropped."""
 
 from __future__ import annotations
 

@@ -364,9 +364,9 @@ def test_packed_train_grads_in_input_dtype(dtype):
 
 
 def test_packed_validation_sees_writes_queued_just_before():
-    """As for the contrastive path: with max_q_len the ids are copied on a
-    side stream that waits for the current one, so an id made invalid just
-    before the call, behind a long kernel, is rejected."""
+    """As for the contrastive path: the check of the ids is queued on the
+    current stream, so an id made invalid just before the call, behind a long
+    kernel, is rejected."""
     q, qoff, d, doff, qids, dids = make_packed(4, 5, 9, 32, (2, 20), (4, 50), torch.float32, seed=8)
     torch.cuda.synchronize()
     a = torch.randn(4096, 4096, device=DEVICE)
