@@ -3042,12 +3042,12 @@ static int packed_backward_impl(
 // gathers that costs it a few ns per document.  Whole backward, fp32, one launch
 // / two, us: dim 64, 8 queries x 64 documents 15 / 20, x 150 46 / 43, x 300 92 /
 // 80, 64 queries x 300 96 / 101; dim 128, 8 x 700 171 / 168, x 2000 727 / 559; dim
-// 256, 8 x 700 193 / 214, x 2000 762 / 680; unaligned rows, dim 300, 8 x 2000 1223
-// / 1744; in bf16 8 x 2000 273 / 322.
+// 256, 8 x 700 193 / 214, x 2000 762 / 680; dim 96 (no bucketing), 2 x 2000 381 /
+// 443; unaligned rows, dim 300, 8 x 2000 1223 / 1744; in bf16 8 x 2000 273 / 322.
 static bool grads_one_launch(maxsim_dtype dtype, bool vec, bool dd_bucket, int64_t rows,
                              int64_t nb, int64_t dim) {
-  if (dtype != MAXSIM_FLOAT32 || !vec) return true;
-  return nb <= (dd_bucket && dim <= 64 ? std::max<int64_t>(128, rows / 4) : 1024);
+  if (dtype != MAXSIM_FLOAT32 || !vec || (!dd_bucket && dim <= 128)) return true;
+  return nb <= (dim <= 64 ? std::max<int64_t>(128, rows / 4) : 1024);
 }
 
 static int contrastive_backward_impl(

@@ -2243,7 +2243,7 @@ static bool kloop_pays(maxsim_dtype dtype, int64_t dim, bool vec, bool copy_d, i
     slot = dim > kMaxRegDim ? 0.375
            : vec            ? (dim > 128 ? 0.7 : 0.75)
                             : (dim > 128 ? 0.25 : 0.5);
-    copy = 2.0;
+    copy = 1.5;
   } else {
     if (dim > kMaxRegDim && work < 3 * cus) return true;  // the wide pair kernel's latency
     slot = dim > kMaxRegDim ? 0.1 : !vec && dim > 128 ? 0.25 : 0.35;

@@ -58,6 +58,7 @@ def test_unfilled_groups_take_the_pair_kernels(route, dtype, dim, nq, lq, nb):
     (F32, 128, 72, 32, 72, KLOOP),
     (F32, 128, 1, 250, 1000, KLOOP),     # 285, 172
     (F32, 72, 6, 32, 4000, KLOOP_WS),    # 540, 391
+    (F32, 72, 9, 32, 4000, KLOOP_WS),    # 762, 627
     (F32, 200, 4, 32, 4000, KLOOP_WS),
     (F32, 384, 8, 32, 1000, KLOOP),
     (BF16, 96, 4, 32, 4000, KLOOP_WS),

@@ -28,6 +28,7 @@ def lib():
     (F32, 1, 1, 256, 2000, 128, 0),   # 727, 559
     (F32, 1, 0, 256, 2000, 256, 0),   # 762, 680
     (F32, 1, 0, 256, 700, 256, 1),    # 193, 214
+    (F32, 1, 0, 64, 2000, 96, 1),     # 381, 443
     (F32, 0, 0, 256, 2000, 300, 1),   # 1223, 1744
     (BF16, 1, 1, 256, 2000, 128, 1),  # 273, 322
     (F16, 1, 1, 256, 2000, 64, 1),
