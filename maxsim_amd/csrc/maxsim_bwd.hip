@@ -838,14 +838,16 @@ constexpr int kDdBatch = 8;      // bucket entries gathered per step
 constexpr int kDdBlock = 32;     // bucket entries per block sum
 constexpr int kDdSortBatch = 8;  // argmax loads in flight per thread while sorting
 
-// Waves per SIMD that dd_contrastive_kernel is compiled for, aligned rows of one
-// slice per lane: four, two workgroups per CU.  Left to itself the compiler
-// takes 129 registers for fp32, one too many: 300 x 300 documents of 20-400
-// rows, dim 200, 253 -> 216 us.  (Not with dq in the launch, where the second
+// Waves per SIMD that dd_contrastive_kernel is compiled for, aligned fp32 rows
+// of one slice per lane: four, two workgroups per CU.  Left to itself the
+// compiler takes 129 registers, one too many: 300 x 300 documents of 20-400
+// rows, dim 200, 253 -> 216 us.  The 16-bit kernels have their four waves and
+// lose by the bound's other schedule (457 queries of 59 tokens x 703 documents,
+// dim 128, whole step 2041 -> 2248 us).  (Not with dq in the launch, where the second
 // workgroup gets in dq's way: whole backward, 30 queries of 20 tokens x 150
 // documents, dim 200, 36 us at three waves, 47 at four.)
-template <bool VEC, int NS>
-constexpr int kDdMinWaves = VEC && NS == 1 ? 4 : 1;
+template <typename T, bool VEC, int NS>
+constexpr int kDdMinWaves = T::bytes == 4 && VEC && NS == 1 ? 4 : 1;
 
 // x / d for 0 <= x < 2^24, d >= 1, from a float reciprocal: x is exact in
 // fp32 and the rounded product is within one of the quotient (exact for
@@ -1078,7 +1080,7 @@ __device__ __forceinline__ void dd_contrastive_document(const DdArgs& a, unsigne
 }
 
 template <typename T, bool VEC, int NS, typename O>
-__global__ __launch_bounds__(kDdThreads, (kDdMinWaves<VEC, NS>)) void dd_contrastive_kernel(
+__global__ __launch_bounds__(kDdThreads, (kDdMinWaves<T, VEC, NS>)) void dd_contrastive_kernel(
     DdArgs a) {
   dd_contrastive_document<T, VEC, NS, O>(a, blockIdx.x);
 }
