@@ -2171,7 +2171,10 @@ constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // 16-bit rows that could be used in place have the queries' fragments put in
 // order (one launch more, about 3 us) from this many operations: 7e9 at dim 96
 // ran 33.1 us without and 36.8 us with it, 2e10 at dim 256 101.9 and 83.6 us;
-// wider rows always;
+// from 320 elements always, if the queries fill their blocks (1 x 1000 documents
+// at dim 768 152 / 122 us, 20 x 150 at dim 320 24.2 / 21.3, 4 x 32 at dim 384
+// 20.5 / 20.6; but 32 queries of 11 tokens x 64 at dim 384 19.8 / 21.9, 8 x 64 at
+// dim 272 16.7 / 18.3);
 // fp32, bound by its MFMAs, gained nothing
 constexpr double kFragMinOps = 1e10;
 
@@ -2276,8 +2279,10 @@ static ContrastiveRoute contrastive_route(maxsim_dtype dtype, const void* q, int
   r.kloop = true;
   r.in_place = dim % kChunk == 0 && ptrs;
   r.copy_d = copy_d;
-  if (r.in_place && (dtype == MAXSIM_FLOAT32 || (dim <= kMaxRegDim &&
-                     2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps)))
+  const bool wide = dim >= 320 && 4 * lq >= 3 * nblk * kTileCols;
+  if (r.in_place &&
+      (dtype == MAXSIM_FLOAT32 ||
+       (!wide && 2.0 * (double)dim * (double)(nq * lq) * (double)total_d < kFragMinOps)))
     return r;
   r.ws = kloop_workspace_bytes(dtype, nq, nblk, total_d, dim, r.copy_d);
   if (r.ws > kMaxWorkspace) r.ws = 0;

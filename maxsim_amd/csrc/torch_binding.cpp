@@ -80,6 +80,26 @@ int64_t check_tag(const int64_t* w, int64_t words) {
   return (int64_t)(reinterpret_cast<uintptr_t>(w) ^ (0x6d617873696d0000ull + (uint64_t)words));
 }
 
+// The words of a check, freed behind an event on its stream if some are not
+// written yet.
+struct CheckWords {
+  at::DataPtr block;
+  c10::Stream stream;
+  int words;
+
+  static void release(void* p) {
+    auto* c = static_cast<CheckWords*>(p);
+    const int64_t* w = static_cast<const int64_t*>(c->block.get());
+    for (int i = 0; i < c->words; ++i) {
+      if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) & 1) continue;
+      at::getHostAllocator(at::kCUDA)->record_event(c->block.get(), c->block.get_context(),
+                                                    c->stream);
+      break;
+    }
+    delete c;
+  }
+};
+
 // Queue the check of a call's index arrays on the current stream, ahead of
 // the call's kernels; the words of the result are for check_wait(), the last
 // two are the stream and a tag that only these results have.  The words are
@@ -119,23 +139,22 @@ Tensor check_begin(const std::vector<std::tuple<Tensor, int, int64_t>>& checks) 
   const Tensor& first = held.front();
   c10::hip::HIPGuardMasqueradingAsCUDA guard(first.device());
   const int words = maxsim_internal_check_words(arrays, n);
-  Tensor pinned =
-      at::empty({words + 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-  int64_t* w = pinned.data_ptr<int64_t>();
+  const size_t bytes = sizeof(int64_t) * (size_t)(words + 2);
+  at::DataPtr pinned = at::getHostAllocator(at::kCUDA)->allocate(bytes);
+  int64_t* w = static_cast<int64_t*>(pinned.get());
   for (int i = 0; i < words; ++i) w[i] = 0;
   void* stream = reinterpret_cast<void*>(s.stream());
   w[words] = reinterpret_cast<intptr_t>(stream);
   w[words + 1] = check_tag(w, words);
   check_status(maxsim_internal_check_layout(arrays, n, reinterpret_cast<uint64_t*>(w), stream));
-  auto release = [pinned, s = s.unwrap(), words](void* p) {
-    const int64_t* v = static_cast<const int64_t*>(p);
-    for (int i = 0; i < words; ++i) {
-      if (__atomic_load_n(v + i, __ATOMIC_ACQUIRE) & 1) continue;
-      at::getHostAllocator(at::kCUDA)->record_event(p, pinned.storage().data_ptr().get_context(), s);
-      break;
-    }
-  };
-  return at::from_blob(w, {words + 2}, std::move(release), at::TensorOptions().dtype(at::kLong));
+  // a tensor over the words (at::from_blob costs a microsecond more)
+  at::DataPtr data(w, new CheckWords{std::move(pinned), s.unwrap(), words}, &CheckWords::release,
+                   at::kCPU);
+  Tensor status = at::detail::make_tensor<c10::TensorImpl>(
+      c10::Storage(c10::Storage::use_byte_size_t(), bytes, std::move(data)),
+      c10::DispatchKeySet(c10::DispatchKey::CPU), caffe2::TypeMeta::Make<int64_t>());
+  status.unsafeGetTensorImpl()->set_sizes_contiguous({words + 2});
+  return status;
 }
 
 Tensor maxsim_check_padded(Tensor query_lengths, Tensor doc_lengths, int64_t Lq, int64_t Ld) {

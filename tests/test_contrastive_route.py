@@ -68,6 +68,8 @@ def test_unfilled_groups_take_the_pair_kernels(route, dtype, dim, nq, lq, nb):
     (BF16, 300, 1, 32, 100, KLOOP_WS),   # 37, 31
     (BF16, 768, 1, 32, 1000, KLOOP_WS),
     (BF16, 768, 64, 32, 64, KLOOP_WS),
+    (BF16, 384, 32, 11, 64, KLOOP),      # queries that fill a third of their blocks
+    (BF16, 272, 8, 32, 64, KLOOP),       # 16.7, 18.3 with the queries in order
     (F32, 64, 10, 77, 1000, TILED),      # 456, 353
     (F32, 64, 9, 250, 64, TILED),        # 161, 77
     (BF16, 64, 3, 77, 1000, TILED),      # 51, 39
