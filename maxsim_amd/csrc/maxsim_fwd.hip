@@ -2211,8 +2211,8 @@ static bool long_queries_tiled(maxsim_dtype dtype, int64_t dim, int64_t nq, int6
     return (double)(nq * nblk) * rounds / (pairs / 4.0) > slot * (double)slots;
   }
   // workgroups beyond one per CU share it
-  const double pair_turns = std::max(1.0, 0.5 + 0.5 * pairs);
-  const double tiled_turns = std::max(1.0, narrow ? wgs : 0.5 + 0.5 * wgs);
+  const double pair_turns = 0.5 + 0.5 * std::ceil(pairs);
+  const double tiled_turns = narrow ? std::ceil(wgs) : 0.5 + 0.5 * std::ceil(wgs);
   return (double)nblk * pair_turns > serial * tiled_turns;
 }
 
