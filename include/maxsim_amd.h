@@ -244,7 +244,11 @@ int maxsim_amd_padded_backward_typed(
 
 /* Replaces op `maxsim_contrastive_forward` (torch_binding.h:133-135,
  * maxsim.cu:1718-1779).  queries [Nq, Lq, dim], documents [total_d_tokens,
- * dim], document_offsets [Nb+1] -> scores [Nq, Nb]. */
+ * dim], document_offsets [Nb+1] -> scores [Nq, Nb].  Rows are read in place:
+ * wide rows that are not whole 16-element chunks on 16-byte boundaries, which
+ * the torch operators first copy into a workspace, take the slower kernels that
+ * score pair by pair here (the same bits).  Padding dim to a multiple of 16
+ * avoids that. */
 int maxsim_amd_contrastive_forward(maxsim_dtype dtype, const void* queries,
                                    int64_t num_queries, int64_t Lq,
                                    const void* documents,

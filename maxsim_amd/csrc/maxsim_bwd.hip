@@ -2205,11 +2205,11 @@ __device__ __forceinline__ bool dd_packed_multi_stage(const PackedBwdArgs& a, in
 // (half the write bytes) the kernel waits on each workgroup's chain of
 // dependent loads, and five workgroups per CU (96 VGPRs, a few spills in the
 // batch-of-8 path) beat four at 106 VGPRs: C4 typed backward 179.6 -> 170.3
-// us.  fp32 rows are bound by their writes, and the same bound cost 10 us
-// there (294.5 -> 304.6 us), so they keep the compiler's allocation, as do
-// unaligned rows (element loads: 148 VGPRs, whose cap would spill 47).
-// (Four waves for fp32 rows: with dq in the same kernel the compiler would
-// take 139 registers for fp32 inputs, three waves.)
+// us.  fp32 rows are bound by their writes, and five waves cost 10 us there
+// (294.5 -> 304.6 us): they are held at four, since with dq in the same kernel
+// the compiler would take 139 registers for fp32 inputs, three waves.
+// Unaligned rows and rows of two slices per lane keep the compiler's allocation
+// (149 registers for the former, whose cap would spill 47).
 template <bool VEC, int NS, typename O>
 constexpr int kPkMinWaves = (VEC && NS == 1) ? (O::bytes == 2 ? 5 : 4) : 1;
 
@@ -3035,7 +3035,7 @@ static int packed_backward_impl(
   const int G = pow2_at_least(nslices < 16 ? nslices : 16);  // lanes per dd row
   const bool vec_g = vec && aligned16b(dqueries) && aligned16b(ddocuments);
   MAXSIM_DISPATCH(dtype, launch_packed_grouped, a, g, vec_g, G, out16, st);
-  return check_launch("grads_packed_kernel");
+  return check_launch("dq_packed_kernel / grads_packed_kernel / dd_packed_multi_kernel");
 }
 
 // Whether dq runs in the dd launch, as far as the documents go (vec: aligned
@@ -3268,14 +3268,14 @@ static int contrastive_backward_impl(
         : dtype == MAXSIM_FLOAT16 ? launch_dd_bucket<F16>(ba, with_dd, blds, out16, st)
                                   : launch_dd_bucket<F32>(ba, with_dd, blds, out16, st);
     if (rc) return rc;
-    return check_launch("dd_bucket_kernel");
+    return check_launch(with_dd ? "grads_bucket_kernel" : "dd_bucket_kernel");
   }
   const int rc =
       dtype == MAXSIM_BFLOAT16 ? launch_dd_contrastive<BF16>(da, with_dd, vec, lds, out16, st)
       : dtype == MAXSIM_FLOAT16 ? launch_dd_contrastive<F16>(da, with_dd, vec, lds, out16, st)
                                 : launch_dd_contrastive<F32>(da, with_dd, vec, lds, out16, st);
   if (rc) return rc;
-  return check_launch("dd_contrastive_kernel");
+  return check_launch(with_dd ? "grads_contrastive_kernel" : "dd_contrastive_kernel");
 }
 
 }  // namespace maxsim

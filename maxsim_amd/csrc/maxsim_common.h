@@ -156,13 +156,14 @@ __device__ __forceinline__ Frag<T> load_frag(const typename T::storage* row,
 // A row's KS chunks (16 elements each, this lane's halves at 8 * h) for the
 // kernels that hold a whole row, by a constant of the launch: aligned whole
 // fragments; rows of at least 8 elements that start anywhere; shorter ones (and
-// fp32 ones of 129 elements and more, for their registers), element by element.  Chunks past the embedding dimension are neither loaded
-// nor (mma_chunks) multiplied.  (Its own constant for the short rows: their
-// loads' many branches would spill scalar registers in every kernel.)  Rows
-// of widths such as 96, 100 or 300 were read element by element before:
-// packed bf16 dim 96, 777 pairs 66 -> 13.5 us; padded fp16 dim 300, 28k pairs
-// 2658 -> 685 us; padded bf16 dim 96, 6400 pairs of up to 300 rows 278 -> 52 us
-// (same bits).
+// fp32 ones of 129 elements and more, for their registers), element by element.
+// Chunks past the embedding dimension are neither loaded nor (mma_chunks)
+// multiplied.  (Its own constant for the short rows: their loads' many branches
+// would add to the scalar spills of every other kernel.)  Rows of widths such as
+// 96, 100 or 300 were read element by element before: packed bf16 dim 96, 777
+// pairs of queries of 38 to 77 tokens 182 -> 28 us; padded fp16 dim 300, 28k
+// pairs 2658 -> 685 us; padded bf16 dim 96, 6400 pairs of up to 300 rows 278 ->
+// 52 us (same bits).
 enum RowLoad : int { kRowShort = 0, kRowVec = 1, kRowAny = 2 };
 template <typename T, int KS, int LOAD>
 __device__ __forceinline__ void load_row(const typename T::storage* row, int h, int dim,

@@ -1,6 +1,7 @@
 // Contrastive forward for rows that contrastive_tiled_kernel does not keep in
-// registers: fp32 above 64 elements, 16-bit rows above 128 or of another
-// width than 32, 64 and 128.
+// registers: of other widths than its own (16-bit 32, 64 and 128, fp32 32 and
+// 64) or off 16-byte boundaries, from 33 fp32 or 65 16-bit elements (two
+// slices) up.
 #include "maxsim_tiled.h"
 
 #include <type_traits>
