@@ -3,7 +3,7 @@
 Tolerances.  The oracle consumes exactly the (rounded) values the kernel
 reads and accumulates in float64, so the only difference left is the
 kernel's fp32 accumulation order.  The bars below are therefore tighter than
-the north-star bounds (1e-5 relative for fp32, 2e-2 for bf16/fp16).
+the contract (1e-5 relative for fp32, 2e-2 for bf16/fp16).
 """
 
 from __future__ import annotations
